@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../host/fl_cell.h"
+#include "../host/fl_copy.h"
 #include "fl_launch.h"
 #include "fletcher/driver.h"
 #include "fletcher/fl_hip.h"
@@ -166,57 +167,175 @@ extern "C" int fl_bytes_per_cell(void)
     return 24 + c;
 }
 
+// ------------------------------------------------------------------ host transfers
+// Host arrays travel in chunks of PIPE_BYTES through two pinned buffers and their device
+// twins: while one chunk crosses the bus and is packed (or unpacked) by a kernel, the host
+// fills (or empties) the other.  Records used to go up through hipMemcpy2D from pageable
+// memory, which the runtime splits into one copy a row: 10 us a row, 330 of the 340 ms of a
+// 128^3 DRIVER_Initialize, now 10 ms; a 384^3 field came down at 17 GB/s in pageable
+// copies (13 ms), now in 4.6 ms.  Kept between transfers, released by DRIVER_Finalize and
+// fl_batch_destroy.
+constexpr size_t PIPE_BYTES = 16u << 20;
+struct Pipe {
+    char *pin[2] = {nullptr, nullptr}, *dev[2] = {nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr};  // the buffer's last use on g_stream
+};
+static Pipe g_pipe;
+
+static void free_xfer()
+{
+    if (g_stream) (void)hipStreamSynchronize(g_stream);
+    for (int b = 0; b < 2; b++) {
+        if (g_pipe.pin[b]) (void)hipHostFree(g_pipe.pin[b]);
+        if (g_pipe.dev[b]) (void)hipFree(g_pipe.dev[b]);
+        if (g_pipe.ev[b]) (void)hipEventDestroy(g_pipe.ev[b]);
+    }
+    g_pipe = Pipe();
+}
+
+// The pipe's buffers, idle.
+static int ensure_pipe()
+{
+    HIPCHK(hipStreamSynchronize(g_stream));
+    if (g_pipe.ev[1]) return FL_OK;
+    long long dummy = 0;
+    for (int b = 0; b < 2; b++) {
+        int rc = dev_alloc((void **)&g_pipe.dev[b], PIPE_BYTES, &dummy);
+        if (!rc && hipHostMalloc((void **)&g_pipe.pin[b], PIPE_BYTES, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            g_pipe.pin[b] = nullptr;
+            rc = fail(FL_ERR_NOMEM, "pinned staging of %zu bytes failed", PIPE_BYTES);
+        }
+        if (!rc && hipEventCreateWithFlags(&g_pipe.ev[b], hipEventDisableTiming) != hipSuccess) {
+            g_pipe.ev[b] = nullptr;
+            rc = fail(FL_ERR_HIP, "event creation failed");
+        }
+        if (rc) {
+            free_xfer();
+            return rc;
+        }
+    }
+    return FL_OK;
+}
+
+// Component fld of a pitched volume of ST values a cell (field_pack) from / to a
+// reference-layout host volume, chunk by chunk through the pipe.
+template <int ST>
+static int volume_xfer(float *vol, int fld, float *host, bool put, int sx, int sy, int sz, int px)
+{
+    const long long n = (long long)sx * sy * sz;
+    const int chunk = (int)(PIPE_BYTES / 4);
+    int rc = ensure_pipe();
+    if (rc) return rc;
+    auto part = [&](long long k) { return (int)std::min<long long>(chunk, n - k * chunk); };
+    const long long nc = (n + chunk - 1) / chunk;
+    hipError_t e = hipSuccess;
+    // getting: chunk k is unpacked and copied while the host empties chunk k - 1
+    for (long long k = 0; k < nc + (put ? 0 : 1) && e == hipSuccess; k++) {
+        const int b = (int)(k & 1);
+        if (k < nc) {
+            const int m = part(k), x0 = (int)(k * chunk % sx);
+            const long long row0 = k * chunk / sx;
+            const dim3 g((m + 255) / 256);
+            float *const dev = (float *)g_pipe.dev[b];
+            if (put) {
+                if (k >= 2) e = hipEventSynchronize(g_pipe.ev[b]);
+                if (e != hipSuccess) break;
+                fl_copy_parallel(g_pipe.pin[b], host + k * chunk, (size_t)m * 4);
+                e = hipMemcpyAsync(dev, g_pipe.pin[b], (size_t)m * 4, hipMemcpyHostToDevice, g_stream);
+                hipLaunchKernelGGL(field_pack<ST>, g, dim3(256), 0, g_stream, dev, vol, fld, m, x0, row0, sx, px);
+            } else {
+                hipLaunchKernelGGL(field_unpack<ST>, g, dim3(256), 0, g_stream, vol, dev, fld, m, x0, row0, sx, px);
+                e = hipMemcpyAsync(g_pipe.pin[b], dev, (size_t)m * 4, hipMemcpyDeviceToHost, g_stream);
+            }
+            if (e == hipSuccess) e = hipGetLastError();
+            if (e == hipSuccess) e = hipEventRecord(g_pipe.ev[b], g_stream);
+        }
+        if (!put && k >= 1 && e == hipSuccess) {
+            e = hipEventSynchronize(g_pipe.ev[b ^ 1]);
+            if (e == hipSuccess) fl_copy_parallel(host + (k - 1) * chunk, g_pipe.pin[b ^ 1], (size_t)part(k - 1) * 4);
+        }
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
+    if (e != hipSuccess) return fail(FL_ERR_HIP, "host transfer: %s", hipGetErrorString(e));
+    return FL_OK;
+}
+
+// One field (fld 0 p, 1 q) of a level.
+static int level_xfer(float *lv, int fld, float *host, bool put, int sx, int sy, int sz, int px)
+{
+    return volume_xfer<2>(lv, fld, host, put, sx, sy, sz, px);
+}
+
+// Records of m cells from their coefficients in consecutive arrays of m (precomp.h order, the
+// 10 coefficients or the 6 recompute inputs), the first one cell x0 of pitched row row0: the
+// slots in the order of rec_order32 / rec_order16 / rec_order_r32 / rec_order_r16, FP32 in
+// its two arrays.  Bound by the bus that feeds it.
+template <int CM>
+__global__ __launch_bounds__(256) void pack_records(const void *soa, int m, int x0, long long row0, int sx, int px,
+                                                    long long np, void *rec)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= m) return;
+    const int r = (x0 + i) / sx, x = x0 + i - r * sx;
+    const long long c = (row0 + r) * px + x;
+    if constexpr (CM == CM_F32) {
+        const float *f = (const float *)soa + i;
+        float v[10];
+#pragma unroll
+        for (int s = 0; s < 10; s++) v[s] = f[(long long)rec_order32(s) * m];
+        float4 *r1 = (float4 *)rec + c * 2;
+        r1[0] = make_float4(v[0], v[1], v[2], v[3]);
+        r1[1] = make_float4(v[5], v[6], v[7], v[8]);
+        ((float2 *)((char *)rec + fp32_part2(np)))[c] = make_float2(v[4], v[9]);
+    } else if constexpr (CM == CM_F32R) {
+        const float *f = (const float *)soa + i;
+        float2 *o = (float2 *)rec + c * 3;
+#pragma unroll
+        for (int s = 0; s < 3; s++)
+            o[s] = make_float2(f[(long long)rec_order_r32(2 * s) * m], f[(long long)rec_order_r32(2 * s + 1) * m]);
+    } else {
+        constexpr bool R = CM == CM_F16R || CM == CM_Q16R;
+        constexpr int NW = R ? 3 : 5;
+        const uint16_t *h = (const uint16_t *)soa + i;
+        uint32_t *o = (uint32_t *)rec + c * NW;
+#pragma unroll
+        for (int s = 0; s < NW; s++) {
+            const int k0 = R ? rec_order_r16(2 * s) : rec_order16(2 * s);
+            const int k1 = R ? rec_order_r16(2 * s + 1) : rec_order16(2 * s + 1);
+            o[s] = (uint32_t)h[(long long)k0 * m] | ((uint32_t)h[(long long)k1 * m] << 16);
+        }
+    }
+}
+
 // Host precompute into the device coefficient records: per cell, its coef_count(cm)
-// values (FP32 or the 16-bit forms, or the recompute inputs) in the slot order
-// rec_order32 / rec_order16 / rec_order_r32 / rec_order_r16 (record of
-// coef_count * coef_elem bytes; FP32 in its two arrays, slots 0-3, 5-8 and slots 4, 9);
-// z slabs of at most 64 MiB per array on the host.
+// values (FP32 or the 16-bit forms, or the recompute inputs), chunk by chunk through the
+// pipe and packed by pack_records.
 // ebase: the CM_Q16R exponent base (fl_recompute_q16_base over the whole grid).
 static int upload_coefs(const float *vpz, const float *vsv, const float *eps, const float *del,
                         const float *phi, const float *theta, float dt, int cm, void *dst, int sx,
                         int sy, int sz, int px, int ebase = 0)
 {
-    const long long sxy = (long long)sx * sy;
-    const int slab = std::max(1, (int)std::min<long long>(sz, (64ll << 20) / (sxy * 4)));
-    const int nk = coef_count(cm);
-    const size_t rec = (size_t)nk * coef_elem(cm);
-    HIPCHK(hipMemset(dst, 0, rec * px * sy * sz));  // pitch padding
-    std::vector<float> f32, r32;
-    std::vector<uint16_t> h16, r16;
-    for (int z0 = 0; z0 < sz; z0 += slab) {
-        const int z1 = std::min(sz, z0 + slab);
-        const long long off = (long long)z0 * sxy, m = (long long)(z1 - z0) * sxy;
+    const long long n = (long long)sx * sy * sz, np = (long long)px * sy * sz;
+    const int nk = coef_count(cm), el = coef_elem(cm);
+    const int chunk = (int)(PIPE_BYTES / (nk * el));
+    int rc = ensure_pipe();
+    if (rc) return rc;
+    HIPCHK(hipMemsetAsync(dst, 0, (size_t)nk * el * np, g_stream));  // pitch padding
+    int b = 0;
+    for (long long off = 0; off < n; off += chunk, b ^= 1) {
+        const int m = (int)std::min<long long>(chunk, n - off);
+        if (off >= 2ll * chunk) HIPCHK(hipEventSynchronize(g_pipe.ev[b]));  // the buffer is free again
         if (cm == CM_F32 || cm == CM_F32R) {
-            f32.resize((size_t)nk * m);
-            r32.resize((size_t)nk * m);
             float *c[10];
-            for (int k = 0; k < nk; k++) c[k] = f32.data() + k * m;
+            for (int k = 0; k < nk; k++) c[k] = (float *)g_pipe.pin[b] + (long long)k * m;
             if (cm == CM_F32)
                 fl_precompute_f32(m, vpz + off, vsv + off, eps + off, del + off, phi + off, theta + off, c);
             else
                 fl_pack_recompute32(m, vpz + off, vsv + off, eps + off, del + off, phi + off, theta + off, c);
-            const float *co[10];
-            for (int k = 0; k < nk; k++) co[k] = c[cm == CM_F32 ? rec_order32(k) : rec_order_r32(k)];
-            if (cm == CM_F32) {  // slots 0-3, 5-8 at 32 B a cell, then slots 4, 9 at 8 B a cell
-                const float *c1[8] = {co[0], co[1], co[2], co[3], co[5], co[6], co[7], co[8]};
-                const float *c2[2] = {co[4], co[9]};
-                const long long np = (long long)px * sy * sz;
-                fl_interleave32(m, 8, c1, r32.data());
-                HIPCHK(hipMemcpy2D((char *)dst + (size_t)z0 * sy * px * 32, px * 32, r32.data(), sx * 32, sx * 32,
-                                   (size_t)sy * (z1 - z0), hipMemcpyHostToDevice));
-                fl_interleave32(m, 2, c2, r32.data());
-                HIPCHK(hipMemcpy2D((char *)dst + fp32_part2(np) + (size_t)z0 * sy * px * 8, px * 8, r32.data(),
-                                   sx * 8, sx * 8, (size_t)sy * (z1 - z0), hipMemcpyHostToDevice));
-            } else {
-                fl_interleave32(m, nk, co, r32.data());
-                HIPCHK(hipMemcpy2D((char *)dst + (size_t)z0 * sy * px * rec, px * rec, r32.data(), sx * rec,
-                                   sx * rec, (size_t)sy * (z1 - z0), hipMemcpyHostToDevice));
-            }
         } else {
-            h16.resize((size_t)nk * m);
-            r16.resize((size_t)nk * m);
             uint16_t *c[10];
-            for (int k = 0; k < nk; k++) c[k] = h16.data() + k * m;
+            for (int k = 0; k < nk; k++) c[k] = (uint16_t *)g_pipe.pin[b] + (long long)k * m;
             if (cm == CM_F16R)
                 fl_pack_recompute16(m, vpz + off, vsv + off, eps + off, del + off, phi + off, theta + off, dt, c);
             else if (cm == CM_Q16R)
@@ -229,22 +348,32 @@ static int upload_coefs(const float *vpz, const float *vsv, const float *eps, co
                 // FP16 velocity factors v^2 dt^2 (coefficients 6-9, or recompute inputs 0-3)
                 // overflow to infinity at 65520: v dt above about 256 m
                 const int k0 = cm == CM_F16 ? 6 : 0;
-                for (int k = k0; k < k0 + 4; k++)
-                    for (long long i = 0; i < m; i++)
+                for (int k = k0; k < k0 + 4; k++) {
+                    unsigned inf = 0;
+                    for (int i = 0; i < m; i++) inf |= (c[k][i] & 0x7c00u) == 0x7c00u;
+                    for (int i = 0; inf && i < m; i++)
                         if ((c[k][i] & 0x7c00u) == 0x7c00u)
                             return fail(FL_ERR_ARG,
                                         "velocity factor v^2 dt^2 of cell %lld exceeds the FP16 range "
                                         "(v dt > 256 m): use FP32, BF16 or block floating-point storage",
-                                        (long long)off + i);
+                                        off + i);
+                }
             }
-            const uint16_t *co[10];
-            for (int k = 0; k < nk; k++)
-                co[k] = c[(cm == CM_F16R || cm == CM_Q16R) ? rec_order_r16(k) : rec_order16(k)];
-            fl_interleave16(m, nk, co, r16.data());
-            HIPCHK(hipMemcpy2D((char *)dst + (size_t)z0 * sy * px * rec, px * rec, r16.data(), sx * rec,
-                               sx * rec, (size_t)sy * (z1 - z0), hipMemcpyHostToDevice));
         }
+        HIPCHK(hipMemcpyAsync(g_pipe.dev[b], g_pipe.pin[b], (size_t)m * nk * el, hipMemcpyHostToDevice, g_stream));
+        const dim3 grid((m + 255) / 256);
+        const int x0 = (int)(off % sx);
+        const long long row0 = off / sx;
+        switch (cm) {
+#define FL_PACK(CMV) \
+    case CMV: hipLaunchKernelGGL(pack_records<CMV>, grid, dim3(256), 0, g_stream, g_pipe.dev[b], m, x0, row0, sx, px, np, dst); break;
+            FL_PACK(CM_F32) FL_PACK(CM_BF16) FL_PACK(CM_F16) FL_PACK(CM_F16R) FL_PACK(CM_F32R) FL_PACK(CM_Q16R)
+#undef FL_PACK
+        }
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipEventRecord(g_pipe.ev[b], g_stream));
     }
+    HIPCHK(hipStreamSynchronize(g_stream));
     return FL_OK;
 }
 
@@ -329,16 +458,7 @@ struct ModelSrc {
     const float *a[6];
     fl_model_slab_fn fill;
     void *user;
-    int sx, sy;
 };
-
-static int model_slab(const ModelSrc &src, int z0, int nzs, float *const *out)
-{
-    if (src.fill) return src.fill(src.user, z0, nzs, out[0], out[1], out[2], out[3], out[4], out[5]);
-    const size_t plane = (size_t)src.sx * src.sy;
-    for (int k = 0; k < 6; k++) memcpy(out[k], src.a[k] + (size_t)z0 * plane, plane * nzs * 4);
-    return 0;
-}
 
 static bool g_device_precompute = false;
 
@@ -348,8 +468,9 @@ extern "C" int fl_set_device_precompute(int on)
     return FL_OK;
 }
 
-// The model streamed to the device in z slabs (pinned staging of at most 6 x 64 MiB), the
-// records of form cm computed there into dst; *vq receives 2^ebase for CM_Q16R.
+// The model brought to the device, whole arrays through the pipe, a callback's in z slabs
+// (pinned staging of at most 6 x 64 MiB), and the records of form cm computed there into dst;
+// *vq receives 2^ebase for CM_Q16R.
 static int device_records(const ModelSrc &src, int cm, int sx, int sy, int sz, int px, float dt, void *dst, float *vq)
 {
     const long long np = (long long)px * sy * sz;
@@ -362,7 +483,7 @@ static int device_records(const ModelSrc &src, int cm, int sx, int sy, int sz, i
     int rc = FL_OK;
     for (int k = 0; k < 6 && rc == FL_OK; k++) rc = dev_alloc((void **)&dv[k], (size_t)np * 4, &dummy);
     if (rc == FL_OK) rc = dev_alloc((void **)&scal, 2 * sizeof(unsigned long long), &dummy);
-    if (rc == FL_OK && hipHostMalloc((void **)&stage, (size_t)6 * slab * plane * 4, hipHostMallocDefault) != hipSuccess) {
+    if (rc == FL_OK && src.fill && hipHostMalloc((void **)&stage, (size_t)6 * slab * plane * 4, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         stage = nullptr;
         rc = fail(FL_ERR_NOMEM, "pinned staging of %lld bytes failed", 6ll * slab * plane * 4);
@@ -370,13 +491,16 @@ static int device_records(const ModelSrc &src, int cm, int sx, int sy, int sz, i
     hipError_t e = hipSuccess;
     for (int k = 0; k < 6 && rc == FL_OK && e == hipSuccess; k++) e = hipMemsetAsync(dv[k], 0, (size_t)np * 4, g_stream);
     if (rc == FL_OK && e == hipSuccess) e = hipMemsetAsync(scal, 0, 2 * sizeof(unsigned long long), g_stream);
+    if (!src.fill)
+        for (int k = 0; k < 6 && rc == FL_OK && e == hipSuccess; k++)
+            rc = volume_xfer<1>(dv[k], 0, const_cast<float *>(src.a[k]), true, sx, sy, sz, px);
     float *h[6];
-    for (int k = 0; k < 6; k++) h[k] = stage + (size_t)k * slab * plane;
-    for (int z0 = 0; z0 < sz && rc == FL_OK && e == hipSuccess; z0 += slab) {
+    for (int k = 0; k < 6; k++) h[k] = stage ? stage + (size_t)k * slab * plane : nullptr;
+    for (int z0 = 0; z0 < sz && src.fill && rc == FL_OK && e == hipSuccess; z0 += slab) {
         const int n = std::min(slab, sz - z0);
         e = hipStreamSynchronize(g_stream);  // the staging buffer is free again
         if (e != hipSuccess) break;
-        if (model_slab(src, z0, n, h)) {
+        if (src.fill(src.user, z0, n, h[0], h[1], h[2], h[3], h[4], h[5])) {
             rc = fail(FL_ERR_ARG, "the model source failed for planes %d..%d", z0, z0 + n - 1);
             break;
         }
@@ -544,54 +668,6 @@ static int ensure_dvol()
     if (rc) return rc;
     HIPCHK(hipMemsetAsync(D.dvx, 0, (size_t)2 * D.np * 4, g_stream));
     HIPCHK(hipMemsetAsync(D.dvy, 0, (size_t)2 * D.np * 4, g_stream));
-    return FL_OK;
-}
-
-// Staging buffer of host transfers: z slabs of one field, at most 64 MiB, kept between
-// transfers (released by DRIVER_Finalize and fl_batch_destroy).
-static float *g_xfer = nullptr;
-static size_t g_xfer_bytes = 0;
-
-static void free_xfer()
-{
-    if (g_xfer) (void)hipFree(g_xfer);
-    g_xfer = nullptr;
-    g_xfer_bytes = 0;
-}
-
-// One field (fld 0 p, 1 q) of a level from / to a reference-layout host volume, slab by
-// slab through the staging buffer.
-static int level_xfer(float *lv, int fld, float *host, bool put, int sx, int sy, int sz, int px)
-{
-    const long long plane = (long long)sx * sy;
-    const int zs = (int)std::max<long long>(1, std::min<long long>(sz, (64ll << 20) / (plane * 4)));
-    const size_t need = (size_t)zs * plane * 4;
-    if (g_xfer_bytes < need) {
-        free_xfer();
-        long long dummy = 0;
-        int rc = dev_alloc((void **)&g_xfer, need, &dummy);
-        if (rc) return rc;
-        g_xfer_bytes = need;
-    }
-    hipError_t e = hipStreamSynchronize(g_stream);
-    for (int z0 = 0; z0 < sz && e == hipSuccess; z0 += zs) {
-        const int nz = std::min(zs, sz - z0);
-        float *slab = lv + 2ll * z0 * sy * px;
-        float *h = host + z0 * plane;
-        const size_t bytes = (size_t)nz * plane * 4;
-        const dim3 g((sx + 255) / 256, sy, nz);
-        if (put) {
-            e = hipMemcpy(g_xfer, h, bytes, hipMemcpyHostToDevice);
-            if (e == hipSuccess) hipLaunchKernelGGL(field_pack, g, dim3(256), 0, g_stream, g_xfer, slab, fld, sx, sy, px);
-            if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
-        } else {
-            hipLaunchKernelGGL(field_unpack, g, dim3(256), 0, g_stream, slab, g_xfer, fld, sx, sy, px);
-            e = hipStreamSynchronize(g_stream);
-            if (e == hipSuccess) e = hipMemcpy(h, g_xfer, bytes, hipMemcpyDeviceToHost);
-        }
-        if (e == hipSuccess) e = hipGetLastError();
-    }
-    if (e != hipSuccess) return fail(FL_ERR_HIP, "field transfer: %s", hipGetErrorString(e));
     return FL_OK;
 }
 
@@ -812,8 +888,6 @@ static int initialize(int sx, int sy, int sz, int bord, float dx, float dy, floa
     memset(&src, 0, sizeof(src));
     const float *a[6] = {vpz, vsv, eps, del, phi, theta};
     for (int k = 0; k < 6; k++) src.a[k] = a[k];
-    src.sx = sx;
-    src.sy = sy;
     return initialize_src(sx, sy, sz, bord, dx, dy, dz, dt, src, pp, pc, qp, qc);
 }
 
@@ -825,8 +899,6 @@ extern "C" int fl_initialize_streamed(int sx, int sy, int sz, int bord, float dx
     memset(&src, 0, sizeof(src));
     src.fill = fill;
     src.user = user;
-    src.sx = sx;
-    src.sy = sy;
     int rc = initialize_src(sx, sy, sz, bord, dx, dy, dz, dt, src, nullptr, nullptr, nullptr, nullptr);
     if (rc == FL_OK) fl_clear_error();
     return rc;

@@ -545,23 +545,26 @@ __global__ void insert_source(float *lv, long long c, float s)
     }
 }
 
-// One field (fld 0 p, 1 q) of a level <-> a volume in the reference layout.
-// grid: (ceil(sx/256), sy, sz); block 256
-__global__ __launch_bounds__(256) void field_pack(const float *__restrict__ lin, float *lv, int fld,
-                                                  int sx, int sy, int px)
+// Component fld of a pitched volume of ST values a cell (a level: ST 2, fld 0 p, 1 q; a model
+// volume: ST 1) <-> m consecutive cells in the reference layout, the first one cell x0 of
+// row row0.  grid: ceil(m/256); block 256
+template <int ST>
+__global__ __launch_bounds__(256) void field_pack(const float *__restrict__ lin, float *vol, int fld, int m, int x0,
+                                                  long long row0, int sx, int px)
 {
-    const int x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= sx) return;
-    const long long row = (long long)blockIdx.z * sy + blockIdx.y;
-    lv[2 * (row * px + x) + fld] = lin[row * sx + x];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= m) return;
+    const int r = (x0 + i) / sx;
+    vol[ST * ((row0 + r) * px + (x0 + i - r * sx)) + fld] = lin[i];
 }
-__global__ __launch_bounds__(256) void field_unpack(const float *__restrict__ lv, float *lin, int fld,
-                                                    int sx, int sy, int px)
+template <int ST>
+__global__ __launch_bounds__(256) void field_unpack(const float *__restrict__ vol, float *lin, int fld, int m, int x0,
+                                                    long long row0, int sx, int px)
 {
-    const int x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= sx) return;
-    const long long row = (long long)blockIdx.z * sy + blockIdx.y;
-    lin[row * sx + x] = lv[2 * (row * px + x) + fld];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= m) return;
+    const int r = (x0 + i) / sx;
+    lin[i] = vol[ST * ((row0 + r) * px + (x0 + i - r * sx)) + fld];
 }
 
 #endif  // FL_NO_AUX_KERNELS

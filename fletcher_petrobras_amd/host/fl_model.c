@@ -10,6 +10,7 @@
 #include <math.h>
 
 #include "fl_cell.h"
+#include "fl_copy.h"
 #include <stdlib.h>
 #include <string.h>
 
@@ -317,4 +318,16 @@ void fl_interleave16(int64_t n, int nk, const uint16_t *const *src, uint16_t *ds
 #pragma omp parallel for schedule(static)
     for (int64_t i = 0; i < n; i++)
         for (int k = 0; k < nk; k++) dst[i * nk + k] = src[k][i];
+}
+
+void fl_copy_parallel(void *dst, const void *src, size_t bytes)
+{
+    const size_t part = 1u << 20;
+    const int64_t n = (int64_t)((bytes + part - 1) / part);
+    /* a few MiB take one thread less time than waking the others may */
+#pragma omp parallel for schedule(static) if (n > 4)
+    for (int64_t k = 0; k < n; k++) {
+        const size_t o = (size_t)k * part;
+        memcpy((char *)dst + o, (const char *)src + o, bytes - o < part ? bytes - o : part);
+    }
 }
