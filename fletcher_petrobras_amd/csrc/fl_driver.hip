@@ -571,12 +571,10 @@ static bool use_pair(int cm, int ty, bool twopass)
 }
 
 // z chunk depth for `tiles` tile columns per plane over nzu planes: the chunk count that
-// minimises (rounds of resident workgroups) x (planes a workgroup streams, zt + 8).  At
-// 384^3 it gives 32x12x188 for FP32 (768 tiles, three rounds of 256) and 32x12x94 for the
-// other forms (1536 tiles, three rounds of 512), the autotuner's choices.
-static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
+// minimises (rounds of the `slots` resident workgroups) x (planes a workgroup streams,
+// zt + lead).
+static int chunk_of(long long tiles, int nzu, long long slots, int lead)
 {
-    const long long slots = (long long)std::max(g_cus, 1) * resident_per_cu(ty, cm, use_pair(cm, ty, false));
     double best = 1e300;
     int bz = nzu;
     for (int nzc = 1; nzc <= 64; nzc++) {
@@ -584,10 +582,19 @@ static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
         if (zt < 8 && nzc > 1) break;
         const int n = (nzu + zt - 1) / zt;
         const long long rounds = (tiles * n + slots - 1) / slots;
-        const double cost = (double)rounds * (zt + 8);
+        const double cost = (double)rounds * (zt + lead);
         if (cost < best * 0.999) { best = cost; bz = zt; }
     }
-    return std::max(1, std::min(std::min(bz, nzu), ztmax));
+    return bz;
+}
+
+// The step kernels' chunk depth.  At 384^3 it gives 32x12x188 for FP32 (768 tiles, three
+// rounds of 256) and 32x12x94 for the other forms (1536 tiles, three rounds of 512), the
+// autotuner's choices.
+static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
+{
+    const long long slots = (long long)std::max(g_cus, 1) * resident_per_cu(ty, cm, use_pair(cm, ty, false));
+    return std::max(1, std::min(std::min(chunk_of(tiles, nzu, slots, 8), nzu), ztmax));
 }
 
 static int default_zt(int sx, int sy, int sz, int bord, int ty)
