@@ -13,7 +13,7 @@
 //
 // Kernels here (the z-marching step kernels are in fl_step.h, fl_step2.h and fl_step_batch.h):
 //   direct_dercross  the reference's direct 64-point DerCross form
-//       (original/derivatives.h:59-68), one thread per (x,y) column.
+//       (original/derivatives.h:59-68), z-marching through LDS planes.
 //   der1_pass        pass 1 of the two-pass form (der1der1/OpenMP/openmp_propagate.c:24-76).
 //   insert_source    p[i] += s, q[i] += s (original/OpenMP/openmp_insertsource.c:7-12).
 //   field_pack / field_unpack   one field between the reference layout and a level.
@@ -323,10 +323,252 @@ struct DirectArgs {
     long long np;         // pitched cells of the grid
     float dxxinv, dyyinv, dzzinv, dxyinv, dxzinv, dyzinv, dt;
     int sx, sy, sz, bord, px, zt;
-    int ntx, nty, nblk;   // tiles of 64 x DX_TY cells along x, y; z chunks of zt planes
+    int ntx, nty, nblk;   // tiles of DX_TX x DX_TY cells along x, y; z chunks of zt planes
     float *trace;
     int rec_iz;
 };
+
+// Four consecutive cells along x of one field: one expression evaluates four derivatives with
+// the same operations in the same order.
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+
+// Der2 of derivatives.h:53 in the reference's association order: g(m) is the values m cells
+// along the axis.
+template <class G>
+__device__ __forceinline__ f4 der2_f4(G g, float d2inv)
+{
+    return (FL_K0 * g(0) + FL_K1 * (g(1) + g(-1)) + FL_K2 * (g(2) + g(-2)) + FL_K3 * (g(3) + g(-3)) +
+            FL_K4 * (g(4) + g(-4))) *
+           d2inv;
+}
+
+// The running sum over the ten coefficient groups of DerCross (derivatives.h:59-68), g(m, n)
+// the sum of group (m, n): the same additions in the same order.
+template <class G>
+__device__ __forceinline__ f4 cross_sum(G g, float dinv)
+{
+    f4 s = FL_L11 * g(1, 1);
+    s = s + FL_L12 * g(1, 2);
+    s = s + FL_L13 * g(1, 3);
+    s = s + FL_L14 * g(1, 4);
+    s = s + FL_L22 * g(2, 2);
+    s = s + FL_L23 * g(2, 3);
+    s = s + FL_L24 * g(2, 4);
+    s = s + FL_L33 * g(3, 3);
+    s = s + FL_L34 * g(3, 4);
+    s = s + FL_L44 * g(4, 4);
+    return s * dinv;
+}
+
+// The 12 values x-4 .. x+7 around four cells (three aligned 16-byte LDS reads): at(u) the
+// four cells displaced by u.
+struct XLine {
+    float w[12];
+    __device__ __forceinline__ explicit XLine(const float *p)
+    {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const f4 v = *(const f4 *)(p + 4 * (k - 1));
+            w[4 * k] = v[0]; w[4 * k + 1] = v[1]; w[4 * k + 2] = v[2]; w[4 * k + 3] = v[3];
+        }
+    }
+    __device__ __forceinline__ f4 at(int u) const { return f4{w[4 + u], w[5 + u], w[6 + u], w[7 + u]}; }
+};
+
+// DerCross whose first axis is x: line(v) points at the own cells displaced by v along the
+// second axis.  Lines +-m feed the first half of the groups (m, n >= m) and the second half of
+// the groups (k < m, m), so each line is read once and every group still adds up in its order:
+// h(n, m) - h(-n, m) - h(n, -m) + h(-n, -m), then for n != m the same with m and n exchanged.
+template <class L>
+__device__ __forceinline__ f4 dercross_x(L line, float dinv)
+{
+    f4 g[5][5];
+#pragma unroll
+    for (int m = 1; m <= 4; m++) {
+        const XLine a(line(m)), b(line(-m));
+#pragma unroll
+        for (int k = 1; k < m; k++) g[k][m] = g[k][m] + a.at(k) - a.at(-k) - b.at(k) + b.at(-k);
+#pragma unroll
+        for (int n = m; n <= 4; n++) g[m][n] = a.at(n) - a.at(-n) - b.at(n) + b.at(-n);
+        __builtin_amdgcn_sched_barrier(0);  // two lines in flight
+    }
+    return cross_sum([&](int m, int n) { return g[m][n]; }, dinv);
+}
+
+// DerCross over an accessor h(a, b): the own cells a along the first axis and b along the second.
+template <class H>
+__device__ __forceinline__ f4 dercross_h(H h, float dinv)
+{
+    return cross_sum(
+        [&](int m, int n) {
+            f4 v = h(n, m) - h(-n, m) - h(n, -m) + h(-n, -m);
+            if (m != n) v = v + h(m, n) - h(-m, n) - h(m, -n) + h(-m, -n);
+            __builtin_amdgcn_sched_barrier(0);
+            return v;
+        },
+        dinv);
+}
+
+// Direct 64-point DerCross form (original/sample.h:32-90) staged through LDS.  A workgroup
+// of 8 waves owns 64 x 16 cells of a z chunk.  A lane forms the derivatives of four
+// consecutive cells of one field (lanes 0-31 p, 32-63 q; 16 lanes a row, two rows a wave);
+// the halves of a wave then exchange them (v_permlane32_swap) so that each lane has both
+// fields of two cells, and update those.  The 9 planes of the stencil (tile + 4-cell halo,
+// one array a field) sit in a ring of DX_NP plane slots; the next plane is loaded before the
+// derivatives and stored after them into the slot that no step of the current plane reads, so
+// one barrier a plane suffices.  Every derivative, the coefficient combination and the
+// leapfrog keep the reference's association order: the results are those of the reference's
+// loop, bit for bit.
+//
+// Bound by VALU issue (573 operations a cell, none of them fused, in the reference's order)
+// with the LDS close behind: a lane reads 131 16-byte values a plane, 1048 bytes a cell with
+// both fields, where one cell a lane with both fields read 217 pairs, 1736 bytes.  That form,
+// which also waited for the next plane's loads at the end of each plane, took 414 us on a
+// 192 x 240 x 216 array and 2141 us on 384^3; this one 217 and 1182 us (the VALU operations
+// alone 116 and 775 us).  The LDS ring holds one workgroup a CU.
+constexpr int DX_TX = 64, DX_TY = 16, DX_NW = DX_TY / 2, DX_NT = 64 * DX_NW, DX_NP = 10;
+constexpr int DX_HX = DX_TX + 8, DX_HY = DX_TY + 8, DX_PL = DX_HX * DX_HY;  // cells per staged plane
+constexpr int DX_NLD = (DX_PL + DX_NT - 1) / DX_NT;                         // staging loads per thread
+constexpr int DX_PER_CU = 1;                                                // resident workgroups a CU
+constexpr uint32_t DX_OOB = 0x80000000u;  // beyond every plane (planes hold < 2^31 bytes)
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dx_rsrc(const void *p, uint32_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ float dx_f(uint32_t v) { return __uint_as_float(v); }
+
+// grid: nblk rounded up to whole XCD rounds; block (64, DX_NW).  Fields are (p, q) pairs at
+// the pitched cell index.
+__global__ __launch_bounds__(DX_NT) __attribute__((amdgpu_waves_per_eu(DX_PER_CU * DX_NW / 4)))
+void direct_dercross(const DirectArgs a)
+{
+    __shared__ __attribute__((aligned(16))) float lds[DX_NP][2][DX_PL];
+    const int t = xcd_remap(blockIdx.x, gridDim.x);
+    if (t >= a.nblk) return;
+    const int tx = t % a.ntx, rest = t / a.ntx, ty = rest % a.nty, tz = rest / a.nty;
+    const int x0 = a.bord + tx * DX_TX, y0 = a.bord + ty * DX_TY;
+    const int zlo = a.bord + tz * a.zt, zhi = min(zlo + a.zt, a.sz - a.bord);
+    const int f0 = zlo - 4;  // first staged plane
+    const int lane = threadIdx.x, wv = uni((int)threadIdx.y), tid = wv * 64 + lane;
+    const int fld = lane >> 5, row = 2 * wv + ((lane >> 4) & 1), c4 = (lane & 15) * 4;
+    const uint32_t pxy = (uint32_t)a.px * (uint32_t)a.sy;
+
+    // the two cells this lane updates, and their byte offsets within a plane of pairs (the
+    // records are at 4 times, and at 1 times, these offsets)
+    const int y = y0 + row, x = x0 + c4 + 2 * fld;
+    uint32_t o8[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+        o8[k] = (x + k < a.sx - a.bord && y < a.sy - a.bord) ? (uint32_t)(y * a.px + x + k) * 8u : DX_OOB;
+
+    // staging: cell e of a staged plane is (row e / DX_HX, column e % DX_HX) of the window
+    // whose corner is (x0 - 4, y0 - 4); cells outside the array read as zero.  Loads are
+    // unconditional (out of range offsets read zero), so the waits for them count exactly.
+    uint32_t goff[DX_NLD];
+#pragma unroll
+    for (int k = 0; k < DX_NLD; k++) {
+        const int e = k * DX_NT + tid, r = e / DX_HX, gx = x0 - 4 + e - r * DX_HX, gy = y0 - 4 + r;
+        goff[k] = (e < DX_PL && gx < a.sx && gy < a.sy) ? (uint32_t)(gy * a.px + gx) * 8u : DX_OOB;
+    }
+    auto fetch = [&](int zp, u2v *v) {  // a plane beyond the array: the last one (not read)
+        const __amdgpu_buffer_rsrc_t rs = dx_rsrc(a.cur + 2ll * min(zp, a.sz - 1) * pxy, pxy * 8u);
+#pragma unroll
+        for (int k = 0; k < DX_NLD; k++) v[k] = __builtin_amdgcn_raw_buffer_load_b64(rs, goff[k], 0, 0);
+    };
+    auto stage = [&](int slot, const u2v *v) {
+#pragma unroll
+        for (int k = 0; k < DX_NLD; k++) {
+            const int e = k * DX_NT + tid;
+            const uint32_t p = v[k][0], q = v[k][1];
+            if (e < DX_PL) {
+                lds[slot][0][e] = dx_f(p);
+                lds[slot][1][e] = dx_f(q);
+            }
+        }
+    };
+    {
+        u2v v[9][DX_NLD];
+#pragma unroll
+        for (int i = 0; i < 9; i++) fetch(f0 + i, v[i]);
+#pragma unroll
+        for (int i = 0; i < 9; i++) stage(i, v[i]);
+    }
+    __syncthreads();
+
+    const int own = (row + 4) * DX_HX + c4 + 4;  // own cells in a staged plane
+    for (int z = zlo; z < zhi; z++) {
+        const int j = z - zlo;
+        u2v nxt[DX_NLD];
+        fetch(z + 5, nxt);
+        // records (slots 0-3, 5-8 and 4, 9) and previous level of the two cells, used at the end
+        const __amdgpu_buffer_rsrc_t r_c1 = dx_rsrc(a.coef + (long long)z * pxy * 8, pxy * 32u);
+        const __amdgpu_buffer_rsrc_t r_c2 =
+            dx_rsrc((const char *)a.coef + fp32_part2(a.np) + (long long)z * pxy * 8, pxy * 8u);
+        const __amdgpu_buffer_rsrc_t r_pv = dx_rsrc(a.prev + 2ll * z * pxy, pxy * 8u);
+        u4v k1[2], k2[2];
+        u2v k3[2], pv[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const uint32_t o32 = o8[k] == DX_OOB ? DX_OOB : o8[k] * 4u;
+            k1[k] = __builtin_amdgcn_raw_buffer_load_b128(r_c1, o32, 0, 0);
+            k2[k] = __builtin_amdgcn_raw_buffer_load_b128(r_c1, o32, 16, 0);
+            k3[k] = __builtin_amdgcn_raw_buffer_load_b64(r_c2, o8[k], 0, 0);
+            pv[k] = __builtin_amdgcn_raw_buffer_load_b64(r_pv, o8[k], 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const float *pl[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) pl[k] = &lds[(j + k) % DX_NP][fld][own];
+        auto v4 = [](const float *p) { return *(const f4 *)p; };
+        // xx, yy, zz, xy, yz, xz and the centre
+        f4 d[7];
+        {
+            const XLine l(pl[4]);
+            d[6] = l.at(0);
+            d[0] = der2_f4([&](int m) { return l.at(m); }, a.dxxinv);
+            d[1] = der2_f4([&](int m) { return m ? v4(pl[4] + m * DX_HX) : d[6]; }, a.dyyinv);
+            __builtin_amdgcn_sched_barrier(0);
+            d[2] = der2_f4([&](int m) { return m ? v4(pl[4 + m]) : d[6]; }, a.dzzinv);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        d[3] = dercross_x([&](int v) { return pl[4] + v * DX_HX; }, a.dxyinv);
+        d[4] = dercross_h([&](int u, int v) { return v4(pl[4 + v] + u * DX_HX); }, a.dyzinv);
+        d[5] = dercross_x([&](int v) { return pl[4 + v]; }, a.dxzinv);
+        __builtin_amdgcn_sched_barrier(0);
+        // lanes 0-31 keep cells 0, 1 and lanes 32-63 cells 2, 3, each with both fields
+        float p[7][2], q[7][2];
+#pragma unroll
+        for (int i = 0; i < 7; i++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float lo = d[i][k], hi = d[i][k + 2];
+                const u2v r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+                const uint32_t rp = r[0], rq = r[1];
+                p[i][k] = dx_f(rp);
+                q[i][k] = dx_f(rq);
+            }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            Coef kc;
+            const u4v ka = k1[k], kb = k2[k];
+            const uint32_t w[10] = {ka[0], ka[1], ka[2], ka[3], k3[k][0], kb[0], kb[1], kb[2], kb[3], k3[k][1]};
+#pragma unroll
+            for (int s = 0; s < 10; s++) kc.c[rec_order32(s)] = dx_f(w[s]);
+            const uint32_t op = pv[k][0], oq = pv[k][1];
+            float np = dx_f(op), nq = dx_f(oq);
+            combine<CM_F32>(kc, a.dt, p[0][k], p[1][k], p[2][k], p[3][k], p[4][k], p[5][k], q[0][k], q[1][k], q[2][k],
+                            q[3][k], q[4][k], q[5][k], p[6][k], q[6][k], np, nq);
+            if (a.trace && z == a.rec_iz && o8[k] != DX_OOB)
+                a.trace[(long long)(y - a.bord) * (a.sx - 2 * a.bord) + (x + k - a.bord)] = np;
+            __builtin_amdgcn_raw_buffer_store_b64(u2v{__float_as_uint(np), __float_as_uint(nq)}, r_pv, o8[k], 0, 0);
+        }
+        stage((j + 9) % DX_NP, nxt);  // the slot that no step of this plane reads
+        __syncthreads();
+    }
+}
 
 // Both fields of a cell, so that one expression evaluates the p and the q derivative with
 // the same operations in the same order.
@@ -337,163 +579,6 @@ __device__ __forceinline__ PQ operator+(PQ a, PQ b) { return {a.p + b.p, a.q + b
 __device__ __forceinline__ PQ operator-(PQ a, PQ b) { return {a.p - b.p, a.q - b.q}; }
 __device__ __forceinline__ PQ operator*(float s, PQ a) { return {s * a.p, s * a.q}; }
 __device__ __forceinline__ PQ operator*(PQ a, float s) { return {a.p * s, a.q * s}; }
-
-// Der2 and DerCross of derivatives.h:53,59-68 in the reference's association order, over an
-// accessor: g(m) is the value m cells along the axis, h(a, b) the value a cells along the
-// first axis (s11) and b along the second (s21).
-template <class G>
-__device__ __forceinline__ PQ der2_a(G g, float d2inv)
-{
-    return (FL_K0 * g(0) + FL_K1 * (g(1) + g(-1)) + FL_K2 * (g(2) + g(-2)) + FL_K3 * (g(3) + g(-3)) +
-            FL_K4 * (g(4) + g(-4))) *
-           d2inv;
-}
-template <class H>
-__device__ __forceinline__ PQ cross_group_a(H h, int m, int n)
-{
-    PQ v = h(n, m) - h(-n, m) - h(n, -m) + h(-n, -m);
-    if (m != n) v = v + h(m, n) - h(-m, n) - h(m, -n) + h(-m, -n);
-    return v;
-}
-template <class H>
-__device__ __forceinline__ PQ dercross_a(H h, float dinv)
-{
-    return (FL_L11 * cross_group_a(h, 1, 1) + FL_L12 * cross_group_a(h, 1, 2) + FL_L13 * cross_group_a(h, 1, 3) +
-            FL_L14 * cross_group_a(h, 1, 4) + FL_L22 * cross_group_a(h, 2, 2) + FL_L23 * cross_group_a(h, 2, 3) +
-            FL_L24 * cross_group_a(h, 2, 4) + FL_L33 * cross_group_a(h, 3, 3) + FL_L34 * cross_group_a(h, 3, 4) +
-            FL_L44 * cross_group_a(h, 4, 4)) *
-           dinv;
-}
-
-// dercross_a as a running sum over the coefficient groups (the same additions in the same
-// order), with compiler barriers after the groups of L13, L23 and L44.
-template <class H>
-__device__ __forceinline__ PQ dercross_runs(H h, float dinv)
-{
-    PQ s = FL_L11 * cross_group_a(h, 1, 1);
-    s = s + FL_L12 * cross_group_a(h, 1, 2);
-    s = s + FL_L13 * cross_group_a(h, 1, 3);
-    asm volatile("" ::: "memory");
-    s = s + FL_L14 * cross_group_a(h, 1, 4);
-    s = s + FL_L22 * cross_group_a(h, 2, 2);
-    s = s + FL_L23 * cross_group_a(h, 2, 3);
-    asm volatile("" ::: "memory");
-    s = s + FL_L24 * cross_group_a(h, 2, 4);
-    s = s + FL_L33 * cross_group_a(h, 3, 3);
-    s = s + FL_L34 * cross_group_a(h, 3, 4);
-    s = s + FL_L44 * cross_group_a(h, 4, 4);
-    asm volatile("" ::: "memory");
-    return s * dinv;
-}
-
-// Direct 64-point DerCross form (original/sample.h:32-90) staged through LDS.  A workgroup
-// of DX_TY waves owns 64 x DX_TY cells of a z chunk; a thread computes both fields of its
-// cell.  The 9 planes of the stencil (tile + 4-cell halo, (p, q) pairs) sit in a ring of
-// DX_NP plane slots; the next plane is stored into the slot that no step of the current plane
-// reads, so one barrier a plane suffices.  Every derivative, the coefficient combination and the
-// leapfrog keep the reference's association order: the results are those of the global-
-// memory form, bit for bit.
-constexpr int DX_TX = 64, DX_TY = 4, DX_NP = 10;
-constexpr int DX_HX = DX_TX + 8, DX_HY = DX_TY + 8, DX_PL = DX_HX * DX_HY;  // pairs per staged plane
-constexpr int DX_NLD = (DX_PL + 64 * DX_TY - 1) / (64 * DX_TY);             // staging loads per thread
-constexpr int DX_PER_CU = (160 * 1024) / (DX_NP * DX_PL * 8);                // resident workgroups a CU
-
-// grid: nblk rounded up to whole XCD rounds; block (64, DX_TY).  Fields are (p, q) pairs at
-// the pitched cell index.
-// DX_PER_CU workgroups a CU (the LDS ring bounds them): DX_PER_CU * DX_TY / 4 waves per SIMD
-__global__ __launch_bounds__(64 * DX_TY) __attribute__((amdgpu_waves_per_eu(DX_PER_CU * DX_TY / 4)))
-void direct_dercross(const DirectArgs a)
-{
-    __shared__ float2 lds[DX_NP][DX_PL];
-    const int t = xcd_remap(blockIdx.x, gridDim.x);
-    if (t >= a.nblk) return;
-    const int tx = t % a.ntx, rest = t / a.ntx, ty = rest % a.nty, tz = rest / a.nty;
-    const int x0 = a.bord + tx * DX_TX, y0 = a.bord + ty * DX_TY;
-    const int zlo = a.bord + tz * a.zt, zhi = min(zlo + a.zt, a.sz - a.bord);
-    const int f0 = zlo - 4;  // first staged plane
-    const int c = threadIdx.x, r = threadIdx.y, tid = r * 64 + c;
-    const int x = x0 + c, y = y0 + r;
-    const bool active = x < a.sx - a.bord && y < a.sy - a.bord;
-    const long long pxy = (long long)a.px * a.sy;
-    const float2 *cur2 = (const float2 *)a.cur;
-
-    // staging: pair e of a staged plane is (row e / DX_HX, column e % DX_HX) of the window
-    // whose corner is (x0 - 4, y0 - 4); cells outside the array read as zero
-    int goff[DX_NLD];  // pitched cell offset within a plane (planes hold < 2^31 cells)
-    bool gok[DX_NLD];
-#pragma unroll
-    for (int k = 0; k < DX_NLD; k++) {
-        const int e = k * 64 * DX_TY + tid;
-        const int row = e / DX_HX, col = e - row * DX_HX;
-        const int gx = x0 - 4 + col, gy = y0 - 4 + row;
-        gok[k] = e < DX_PL && gx < a.sx && gy < a.sy;
-        goff[k] = gy * a.px + gx;
-    }
-    auto fetch = [&](int zp, float2 *v) {
-        const float2 *pl = cur2 + zp * pxy;
-#pragma unroll
-        for (int k = 0; k < DX_NLD; k++) v[k] = (gok[k] && zp < a.sz) ? pl[goff[k]] : make_float2(0.f, 0.f);
-    };
-    auto stage = [&](int slot, const float2 *v) {
-#pragma unroll
-        for (int k = 0; k < DX_NLD; k++) {
-            const int e = k * 64 * DX_TY + tid;
-            if (e < DX_PL) lds[slot][e] = v[k];
-        }
-    };
-    for (int i = 0; i < 9; i++) {
-        float2 v[DX_NLD];
-        fetch(f0 + i, v);
-        stage(i, v);
-    }
-    __syncthreads();
-
-    const int own = (r + 4) * DX_HX + (c + 4);  // own cell in a staged plane
-    for (int z = zlo; z < zhi; z++) {
-        const int j = z - zlo;
-        if (active) {
-            const float2 *pl[9];
-#pragma unroll
-            for (int k = 0; k < 9; k++) pl[k] = &lds[(j + k) % DX_NP][own];
-            // both fields at once (8-byte LDS reads), one derivative after the other and the
-            // cross derivatives in three runs of coefficient groups, with compiler barriers
-            // between them: at most 24 pairs of stencil values are live at once
-            auto at = [](const float2 *b, int o) { const float2 v = b[o]; return PQ{v.x, v.y}; };
-            const PQ xx = der2_a([&](int m) { return at(pl[4], m); }, a.dxxinv);
-            const PQ yy = der2_a([&](int m) { return at(pl[4], m * DX_HX); }, a.dyyinv);
-            const PQ zz = der2_a([&](int m) { return at(pl[4 + m], 0); }, a.dzzinv);
-            asm volatile("" ::: "memory");
-            const PQ xy = dercross_runs([&](int u, int v) { return at(pl[4], u + v * DX_HX); }, a.dxyinv);
-            const PQ yz = dercross_runs([&](int u, int v) { return at(pl[4 + v], u * DX_HX); }, a.dyzinv);
-            const PQ xz = dercross_runs([&](int u, int v) { return at(pl[4 + v], u); }, a.dxzinv);
-            const long long cell = (long long)z * pxy + (long long)y * a.px + x;
-            const float4 *r1 = (const float4 *)(a.coef + cell * 8);  // slots 0-3, 5-8
-            const float2 r2 = ((const float2 *)((const char *)a.coef + fp32_part2(a.np)))[cell];  // 4, 9
-            const float4 u = r1[0], w = r1[1];
-            Coef k;
-            k.c[rec_order32(0)] = u.x; k.c[rec_order32(1)] = u.y;
-            k.c[rec_order32(2)] = u.z; k.c[rec_order32(3)] = u.w;
-            k.c[rec_order32(4)] = r2.x;
-            k.c[rec_order32(5)] = w.x; k.c[rec_order32(6)] = w.y;
-            k.c[rec_order32(7)] = w.z; k.c[rec_order32(8)] = w.w;
-            k.c[rec_order32(9)] = r2.y;
-            float2 *pv = (float2 *)a.prev + cell;
-            float2 o = *pv;
-            const PQ cc = {pl[4][0].x, pl[4][0].y};
-            combine<CM_F32>(k, a.dt, xx.p, yy.p, zz.p, xy.p, yz.p, xz.p, xx.q, yy.q, zz.q, xy.q, yz.q, xz.q,
-                            cc.p, cc.q, o.x, o.y);
-            if (a.trace && z == a.rec_iz)
-                a.trace[(long long)(y - a.bord) * (a.sx - 2 * a.bord) + (x - a.bord)] = o.x;
-            *pv = o;
-        }
-        if (z + 5 <= zhi + 3) {  // the next plane into the slot no step of this plane reads
-            float2 nxt[DX_NLD];
-            fetch(z + 5, nxt);
-            stage((j + 9) % DX_NP, nxt);
-        }
-        __syncthreads();
-    }
-}
 
 // ---------------------------------------------------------------------------------
 // Pass 1 of the two-pass form: Dx of pc,qc over ix in [bord, sx-bord), all iy;
