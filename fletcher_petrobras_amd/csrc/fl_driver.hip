@@ -59,7 +59,7 @@ extern "C" void fl_clear_error(void)
 // ------------------------------------------------------------------ helpers
 // ------------------------------------------------------------------ state
 struct Tiles {
-    int ty = 12, zt = 0;  // zt 0: chunk_depth's choice for the grid
+    int ty = 12, zt = 0;  // zt 0: chunk_depth's choice for the grid; (12, 0): pick_shape's
     int hints = 0;        // streaming cache hints of the z-marching step (fl_set_stream_hints)
     int sw = 0;           // tile columns per strip (fl_set_tile_strip); 0: strip_width's choice
     int pair = 1;         // both fields per lane for the forms that have it (fl_set_lane_pairs)
@@ -83,6 +83,8 @@ struct Device {
     float *src_tab = nullptr;  // source samples of the current multi-step run
     int src_cap = 0;
     long long bytes = 0;
+    int auto_form = -1;     // variant and lane layout that the default tiles below are for
+    int auto_ty = 0, auto_zt = 0;
 };
 
 static Device D;
@@ -597,11 +599,91 @@ static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
     return std::max(1, std::min(std::min(chunk_of(tiles, nzu, slots, 8), nzu), ztmax));
 }
 
-static int default_zt(int sx, int sy, int sz, int bord, int ty)
+// Tile rows and chunk depth of the default setting (12 rows, depth 0) for a set of grids stepped
+// together.  The modelled time of a shape, in us, is the 4.5-norm of
+//   marching: rounds of resident workgroups x (zt + 0.46 x 8 lead planes) x the time of a plane
+//     step, 0.45 + 0.038 per wave on the CU (0.71 + 0.044 with both fields per lane): a wave's
+//     own chain of LDS reads and sums, and the issue slots of the others; the last round
+//     with the waves it has;
+//   memory: the step's bytes, the x-y halo and (8 planes a chunk) the z halo, at 6.2 TB/s.
+// Fitted on 15 grids from 28^3 to 376^3 updated cells in FP32, FP32 recompute, FP16, block
+// floating point and the two-pass form, every shape timed: the shape it picks takes 1.0% more
+// than the fastest one on average, 7% at most.  Against 12 rows with chunk_depth (the
+// default before) it is up to twice as fast on small grids (52 x 44 x 40 FP32 15.2 -> 9.0 us,
+// 120^3 28.0 -> 26.0, q16r 27.3 -> 24.4), 10-20% on middle ones (160^3 FP32 58.0 -> 47.7,
+// q16r 248^3 155.7 -> 137.8) and equal or up to 10% faster on large ones; a one-field-per-lane
+// shape has to promise 2% over the 12-row one to replace it (376^3 FP32: 32x16x63 took 735 us
+// against 704).
+struct Shape {
+    int ty, zt;
+};
+struct GridDims {
+    int sx, sy, sz;
+};
+
+static double shape_us(const std::vector<GridDims> &g, int bord, int ty, int zt, int cm, bool twopass)
 {
-    const long long tiles = (long long)tiles_x(sx, bord) * ((sy - 2 * bord + ty - 1) / ty);
+    const bool pair = use_pair(cm, ty, twopass);
+    const int res = resident_per_cu(ty, cm, pair), waves = pair ? ty / 2 : ty;
+    double items = 0, bytes = 0;
+    const double per = 24 + coef_count(cm) * coef_elem(cm) + (twopass ? 32 : 0);
+    for (const GridDims &d : g) {
+        const int nx = d.sx - 2 * bord, ny = d.sy - 2 * bord, nz = d.sz - 2 * bord;
+        const int nzc = (nz + zt - 1) / zt;
+        items += (double)tiles_x(d.sx, bord) * ((ny + ty - 1) / ty) * nzc;
+        bytes += (double)nx * ny * nz * (per + 64.0 * (2.1 * nzc / nz + 1.1 / ty));
+    }
+    const double cus = std::max(1, g_cus / 8), n8 = std::ceil(items / 8);  // per XCD
+    const double full = std::floor(n8 / (cus * res)), rest = std::ceil((n8 - full * cus * res) / cus);
+    const double t0 = pair ? 0.71 : 0.45, tw = pair ? 0.044 : 0.038, steps = zt + 0.46 * 8;
+    double march = full * steps * (t0 + tw * waves * res);
+    if (rest > 0) march += steps * (t0 + tw * waves * rest);
+    return std::pow(std::pow(march, 4.5) + std::pow(bytes / 6.2e6, 4.5), 1 / 4.5);
+}
+
+static Shape pick_shape(const std::vector<GridDims> &g, int bord, int cm, bool twopass)
+{
+    int nzu = 0, ztmax = 1 << 30;
+    for (const GridDims &d : g) {
+        nzu = std::max(nzu, d.sz - 2 * bord);
+        ztmax = std::min(ztmax, max_zt(pitch_of(d.sx), d.sy));
+    }
+    long long tiles = 0;
+    for (const GridDims &d : g) tiles += (long long)tiles_x(d.sx, bord) * ((d.sy - 2 * bord + 11) / 12);
+    Shape best = {12, chunk_depth(tiles, nzu, 12, cm, ztmax)};
+    double least = shape_us(g, bord, best.ty, best.zt, cm, twopass);
+    if (!has_pair_form(cm) && !twopass) least *= 0.98;
+    for (int ty : {4, 8, 12, 16})
+        for (int nzc = 1; nzc <= 64; nzc++) {
+            const int zt = std::min((nzu + nzc - 1) / nzc, ztmax);
+            if (zt < 2 && nzc > 1) break;
+            const double t = shape_us(g, bord, ty, zt, cm, twopass);
+            if (t < least) {
+                least = t;
+                best = {ty, zt};
+            }
+        }
+    return best;
+}
+
+// The tiles the initialised grid's step runs with.
+static Shape grid_shape()
+{
     const int cm = g_variant == FL_VARIANT_FUSED ? D.cm : CM_F32;
-    return chunk_depth(tiles, sz - 2 * bord, ty, cm, max_zt(pitch_of(sx), sy));
+    const int nz = D.sz - 2 * D.bord, ztmax = max_zt(D.px, D.sy);
+    if (g_tiles.zt > 0) return {g_tiles.ty, std::min(std::min(g_tiles.zt, nz), ztmax)};
+    if (g_tiles.ty != 12) {
+        const long long tiles = (long long)tiles_x(D.sx, D.bord) * ((D.sy - 2 * D.bord + g_tiles.ty - 1) / g_tiles.ty);
+        return {g_tiles.ty, chunk_depth(tiles, nz, g_tiles.ty, cm, ztmax)};
+    }
+    const int form = 2 * g_variant + g_tiles.pair;
+    if (D.auto_form != form) {
+        const Shape s = pick_shape({{D.sx, D.sy, D.sz}}, D.bord, cm, g_variant == FL_VARIANT_TWOPASS);
+        D.auto_form = form;
+        D.auto_ty = s.ty;
+        D.auto_zt = s.zt;
+    }
+    return {D.auto_ty, D.auto_zt};
 }
 
 // Tile columns per strip of the workgroup order (tile_of in the kernels).  Tiles that run
@@ -653,9 +735,8 @@ static StepArgs base_args()
     a.dzinv = 1.0f / D.dz;
     a.dt = D.dt;
     a.vq = D.vq;
-    const int zt = g_tiles.zt > 0 ? std::min(std::min(g_tiles.zt, D.sz - 2 * D.bord), max_zt(D.px, D.sy))
-                                  : default_zt(D.sx, D.sy, D.sz, D.bord, g_tiles.ty);
-    fill_geom(a, D.sx, D.sy, D.sz, D.bord, g_tiles.ty, zt);
+    const Shape t = grid_shape();
+    fill_geom(a, D.sx, D.sy, D.sz, D.bord, t.ty, t.zt);
     a.sw = g_tiles.sw > 0 ? std::min(g_tiles.sw, a.ntx) : strip_width(a.ntx);
     a.src_idx = -1;
     a.trace = D.trace;
@@ -683,7 +764,7 @@ static int launch_step(StepArgs a, int it_host, hipStream_t s)
 {
     a.it_host = it_host;
     if (g_variant == FL_VARIANT_FUSED) {
-        return launch_steps(a, g_tiles.ty, D.cm, false, s);
+        return launch_steps(a, grid_shape().ty, D.cm, false, s);
     }
     if (D.cm != CM_F32)
         return fail(FL_ERR_ARG, "variant %d needs FP32 coefficients", g_variant);
@@ -695,7 +776,7 @@ static int launch_step(StepArgs a, int it_host, hipStream_t s)
         dim3 g1((D.sx + 63) / 64, (D.sy + 3) / 4, D.sz);
         hipLaunchKernelGGL(der1_pass, g1, dim3(64, 4), 0, s, a.cur, D.dvx, D.dvy, D.sx, D.sy, D.px,
                            D.bord, a.dxinv, a.dyinv);
-        return launch_steps(a, g_tiles.ty, CM_F32, true, s);
+        return launch_steps(a, grid_shape().ty, CM_F32, true, s);
     }
     if (g_variant == FL_VARIANT_DIRECT) {
         DirectArgs d;
@@ -1083,8 +1164,9 @@ extern "C" int fl_get_lane_pairs(void) { return g_tiles.pair; }
 
 extern "C" int fl_get_tiles(int *ty, int *zt)
 {
-    if (ty) *ty = g_tiles.ty;
-    if (zt) *zt = (g_tiles.zt > 0 || !D.init) ? g_tiles.zt : default_zt(D.sx, D.sy, D.sz, D.bord, g_tiles.ty);
+    const Shape t = D.init ? grid_shape() : Shape{g_tiles.ty, g_tiles.zt};
+    if (ty) *ty = t.ty;
+    if (zt) *zt = g_tiles.zt > 0 ? g_tiles.zt : t.zt;
     return FL_OK;
 }
 
@@ -1176,8 +1258,9 @@ template <class F>
 static int step_graph(int K, F &&args, GraphSlot **out)
 {
     const StepArgs a0 = args(0), a1 = args(1);
+    const int ty = grid_shape().ty;
     for (auto &g : g_graphs)
-        if (g.exec && g.K == K && g.ty == g_tiles.ty && g.cm == D.cm && g.hints == g_tiles.hints &&
+        if (g.exec && g.K == K && g.ty == ty && g.cm == D.cm && g.hints == g_tiles.hints &&
             g.variant == g_variant && g.pair == g_tiles.pair && memcmp(&g.a0, &a0, sizeof(StepArgs)) == 0 &&
             memcmp(&g.a1, &a1, sizeof(StepArgs)) == 0) {
             g.used = ++g_graph_tick;
@@ -1194,7 +1277,7 @@ static int step_graph(int K, F &&args, GraphSlot **out)
     const int lc0 = D.lc;
     int rc = FL_OK;
     for (int k = 0; k < K && rc == FL_OK; k++) {
-        rc = launch_steps(args(k), g_tiles.ty, D.cm, false, g_stream);
+        rc = launch_steps(args(k), ty, D.cm, false, g_stream);
         swap_levels();
     }
     D.lc = lc0;  // K is even: the levels are back in their roles after a replay
@@ -1214,7 +1297,7 @@ static int step_graph(int K, F &&args, GraphSlot **out)
     g->exec = exec;
     g->graph = graph;
     g->K = K;
-    g->ty = g_tiles.ty;
+    g->ty = ty;
     g->cm = D.cm;
     g->hints = g_tiles.hints;
     g->variant = g_variant;
@@ -1291,7 +1374,7 @@ extern "C" int fl_run_steps(int it0, int nsteps, int iSource, const float *src, 
         done = reps * K;
     }
     for (int k = done; k < nsteps; k++) {
-        int rc = launch_steps(step_args(k), g_tiles.ty, D.cm, false, g_stream);
+        int rc = launch_steps(step_args(k), grid_shape().ty, D.cm, false, g_stream);
         if (rc) return rc;
         swap_levels();
     }
@@ -1330,7 +1413,7 @@ extern "C" int fl_run_steps_static(int it0, int nsteps, int iSource, const float
             hipLaunchKernelGGL(insert_source, dim3(1), dim3(64), 0, g_stream, D.lv[D.lc], psrc, src[k]);
             StepArgs a = base_args();
             a.it_host = it0 + 1 + k;
-            int rc = launch_steps(a, g_tiles.ty, D.cm, false, g_stream);
+            int rc = launch_steps(a, grid_shape().ty, D.cm, false, g_stream);
             if (rc) return rc;
             swap_levels();
         }
@@ -1344,7 +1427,7 @@ extern "C" int fl_run_steps_static(int it0, int nsteps, int iSource, const float
             a.par = k & 1;
             a.src_tab = tab;
             a.src_idx = psrc;
-            int rc = launch_steps(a, g_tiles.ty, D.cm, false, g_stream);
+            int rc = launch_steps(a, grid_shape().ty, D.cm, false, g_stream);
             if (rc) return rc;
             swap_levels();
         }
@@ -1533,6 +1616,7 @@ extern "C" int fl_autotune(int steps, const char *cache_path)
     const Tiles keep = g_tiles;
     double best = 1e30;
     Tiles bt = keep;
+    const Shape model = pick_shape({{D.sx, D.sy, D.sz}}, D.bord, D.cm, g_variant == FL_VARIANT_TWOPASS);
     // two passes over the candidates, the fastest single measurement wins: one pass
     // leaves the early candidates timed while the clocks still ramp.  Each is timed with
     // and without the streaming hints.
@@ -1540,7 +1624,9 @@ extern "C" int fl_autotune(int steps, const char *cache_path)
     for (int pass = 0; pass < 2 && rc == FL_OK; pass++)
     for (int ch = 0; ch < nh && rc == FL_OK; ch++)
     for (int cty : {4, 8, 12, 16}) {
-        for (int czt : zt_candidates(std::min(D.sz - 2 * D.bord, max_zt(D.px, D.sy)))) {
+        std::vector<int> depths = zt_candidates(std::min(D.sz - 2 * D.bord, max_zt(D.px, D.sy)));
+        if (cty == model.ty) depths.push_back(model.zt);
+        for (int czt : depths) {
             g_tiles.ty = cty;
             g_tiles.zt = czt;
             g_tiles.hints = ch;

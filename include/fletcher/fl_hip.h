@@ -64,7 +64,9 @@ int fl_set_sync(int on);           /* 1 (default): DRIVER_Propagate waits for th
 
 /* Tile shape of the z-marching kernel: ty rows (4, 8, 12 or 16) of 32 cells, z chunks of
  * zt planes.  zt 0 selects the chunk depth that fits whole rounds of resident workgroups
- * to the grid (the default, with 12-row tiles). */
+ * to the grid; (12, 0), the default, leaves both rows and depth to the grid's size and form.
+ * Results are identical for every shape.  fl_get_tiles returns the shape in use on the
+ * initialised grid. */
 int fl_set_tiles(int ty, int zt);
 int fl_get_tiles(int *ty, int *zt);
 
