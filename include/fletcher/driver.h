@@ -10,7 +10,8 @@
  *    (fl_hip.h), and uploads them with the fields to the GPU.  It reads
  *    pp/pc/qp/qc once (the reference front-end passes zeros).
  *  - DRIVER_InsertSource adds src to the device pc and qc at iSource
- *    (OpenMP/openmp_insertsource.c:7-12, CUDA/cuda_insertsource.cu:28-32).
+ *    (OpenMP/openmp_insertsource.c:7-12, CUDA/cuda_insertsource.cu:28-32), in order with the
+ *    other calls; it does not wait for the device.
  *  - DRIVER_Propagate advances one time step on the device and swaps the device
  *    time levels internally (CUDA/cuda_propagate.cu:37-80); the host pointers are
  *    not touched.  It returns after the step completes, unless fl_set_sync(0).
