@@ -613,7 +613,7 @@ static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
 // 120^3 28.0 -> 26.0, q16r 27.3 -> 24.4), 10-20% on middle ones (160^3 FP32 58.0 -> 47.7,
 // q16r 248^3 155.7 -> 137.8) and equal or up to 10% faster on large ones; a one-field-per-lane
 // shape has to promise 2% over the 12-row one to replace it (376^3 FP32: 32x16x63 took 735 us
-// against 704).
+// against 704; two-pass: 32x16x94 1270 against 1245).
 struct Shape {
     int ty, zt;
 };
@@ -652,7 +652,7 @@ static Shape pick_shape(const std::vector<GridDims> &g, int bord, int cm, bool t
     for (const GridDims &d : g) tiles += (long long)tiles_x(d.sx, bord) * ((d.sy - 2 * bord + 11) / 12);
     Shape best = {12, chunk_depth(tiles, nzu, 12, cm, ztmax)};
     double least = shape_us(g, bord, best.ty, best.zt, cm, twopass);
-    if (!has_pair_form(cm) && !twopass) least *= 0.98;
+    if (!has_pair_form(cm)) least *= 0.98;
     for (int ty : {4, 8, 12, 16})
         for (int nzc = 1; nzc <= 64; nzc++) {
             const int zt = std::min((nzu + nzc - 1) / nzc, ztmax);
@@ -773,9 +773,10 @@ static int launch_step(StepArgs a, int it_host, hipStream_t s)
         if (rc) return rc;
         a.dvx = D.dvx;
         a.dvy = D.dvy;
-        dim3 g1((D.sx + 63) / 64, (D.sy + 3) / 4, D.sz);
-        hipLaunchKernelGGL(der1_pass, g1, dim3(64, 4), 0, s, a.cur, D.dvx, D.dvy, D.sx, D.sy, D.px,
-                           D.bord, a.dxinv, a.dyinv);
+        const int nbx = ((D.sx + 1) / 2 * ((D.sy + D1_ROWS - 1) / D1_ROWS) + 255) / 256;
+        const unsigned nb1 = (unsigned)(((long long)nbx * D.sz + 7) / 8 * 8);
+        hipLaunchKernelGGL(der1_pass, dim3(nb1), dim3(256), 0, s, a.cur, D.dvx, D.dvy, D.sx, D.sy, D.sz, D.px,
+                           D.bord, nbx, a.dxinv, a.dyinv);
         return launch_steps(a, grid_shape().ty, CM_F32, true, s);
     }
     if (g_variant == FL_VARIANT_DIRECT) {
