@@ -441,7 +441,10 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
     // TWOPASS: first-derivative pair volumes of pass 1, over the chunk's input planes
     const __amdgpu_buffer_rsrc_t r_dx = span_rsrc(TWOPASS ? a.dvx + 2 * zin : a.cur, (uint32_t)(nz + 8) * pb8);
     const __amdgpu_buffer_rsrc_t r_dy = span_rsrc(TWOPASS ? a.dvy + 2 * zin : a.cur, (uint32_t)(nz + 8) * pb8);
-    uint32_t dxo[NH];  // this wave's y-halo rows of Dx
+    // Dx of the own cell, of tile rows beyond the update domain too (Dxy of the rows below
+    // reads them), and of this wave's y-halo rows
+    const uint32_t dxc = (x < a.sx && y < a.sy) ? col * 8u + fld * 4u : FL_OOB;
+    uint32_t dxo[NH];
 #pragma unroll
     for (int m = 0; m < NH; m++) {
         const int j = wv + m * TY, gy = y0 - 4 + (j < 4 ? j : TY + j);
@@ -453,7 +456,7 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
     auto fetch_dv = [&](auto Sc, int i) {
         constexpr int S = decltype(Sc)::value;
         const uint32_t so = pin(i) * pb8;
-        dvx_[S] = __builtin_bit_cast(float, bload32(r_dx, vo8, so));
+        dvx_[S] = __builtin_bit_cast(float, bload32(r_dx, dxc, so));
         dvy_[S] = __builtin_bit_cast(float, bload32(r_dy, vo8, so));
 #pragma unroll
         for (int m = 0; m < NH; m++)

@@ -1,5 +1,7 @@
-"""The two-pass form at the edges of pass 1 (two cells and four rows a thread): the derivative volumes
-against the same FP32 operations in numpy, bit for bit, zero outside their ranges.  Odd row lengths, an odd border (a store of one cell at each end), rows not a multiple of four, a single
+"""The two-pass form at the edges of pass 1 (two cells and four rows a thread) and of the loads pass 2
+makes ahead: the derivative volumes against the same FP32 operations in numpy, bit for bit, zero
+outside their ranges, and one step over tile heights and chunk depths of a plane and more.  Odd row
+lengths, an odd border (a store of one cell at each end), rows not a multiple of four, a single
 updated plane, unequal spacings."""
 import numpy as np
 import pytest
@@ -26,7 +28,7 @@ def der1(f, axis, h):
     ((70, 30, 5), 7, (9.0, 12.5, 11.0)),
     ((259, 3, 2), 5, (12.5, 12.5, 12.5)),
 ])
-def test_volumes(fl, dom, bord, d):
+def test_volumes_and_tiles(fl, dom, bord, d):
     nx, ny, nz = dom
     shape = (nz + 2 * bord, ny + 2 * bord, nx + 2 * bord)
     r = np.random.RandomState(nx)
@@ -36,7 +38,8 @@ def test_volumes(fl, dom, bord, d):
     sz, sy, sx = shape
     in_x = (slice(None), slice(None), slice(bord, sx - bord))
     in_y = (slice(None), slice(bord, sy - bord), slice(bord, sx))
-    for tiles in ((12, 0), (4, 1)):
+    first = None
+    for tiles in ((12, 0), (4, 1), (8, 3), (16, 0)):
         g = fl.Driver(variant="twopass", tiles=tiles)
         g.initialize(shape, d, DT, m, fields=fields, bord=bord)
         g.propagate(1)
@@ -44,4 +47,9 @@ def test_volumes(fl, dom, bord, d):
             ref = np.zeros(shape, np.float32)
             ref[rng] = der1(fields[f], ax, d[2 - ax])[rng]
             assert np.array_equal(g.derivative_volume(k), ref), (tiles, k)
+        got = [g.field(k) for k in ("pc", "qc")]
         g.finalize()
+        assert not np.array_equal(got[0], fields[0])
+        first = first or got
+        for a, b in zip(got, first):
+            assert np.array_equal(a, b), tiles
