@@ -1324,7 +1324,12 @@ extern "C" int fl_run_steps(int it0, int nsteps, int iSource, const float *src, 
     const int siz = (int)(iSource / sxy), siy = (int)((iSource % sxy) / D.sx), six = (int)(iSource % D.sx);
     const bool src_in_domain = siz >= D.bord && siz < D.sz - D.bord && siy >= D.bord &&
                                siy < D.sy - D.bord && six >= D.bord && six < D.sx - D.bord;
-    if (g_variant != FL_VARIANT_FUSED || graph_chunk <= 0 || !src_in_domain) {
+    // The two-pass step adds the next source sample itself as well, in plain launches (a step is
+    // longer than its launches), unless steps are timed one by one (fl_set_timing): 70 x 76 x 72
+    // array 18.5 -> 17.0 us a step, 104 x 110 x 100 29.5 -> 28.3, 224 x 208 x 192 168 -> 167.
+    const bool fused = g_variant == FL_VARIANT_FUSED;
+    const bool in_step = fused || (g_variant == FL_VARIANT_TWOPASS && D.cm == CM_F32 && !g_timing);
+    if (!in_step || graph_chunk <= 0 || !src_in_domain) {
         // plain launches: InsertSource + Propagate per step
         const bool sync = g_sync;
         g_sync = false;
@@ -1368,7 +1373,7 @@ extern "C" int fl_run_steps(int it0, int nsteps, int iSource, const float *src, 
         return a;
     };
     int done = 0;
-    if (K >= 2 && nsteps >= K) {
+    if (fused && K >= 2 && nsteps >= K) {
         GraphSlot *g = nullptr;
         int rc = step_graph(K, step_args, &g);
         if (rc) return rc;
@@ -1377,7 +1382,7 @@ extern "C" int fl_run_steps(int it0, int nsteps, int iSource, const float *src, 
         done = reps * K;
     }
     for (int k = done; k < nsteps; k++) {
-        int rc = launch_steps(step_args(k), grid_shape().ty, D.cm, false, g_stream);
+        int rc = launch_step(step_args(k), 0, g_stream);
         if (rc) return rc;
         swap_levels();
     }

@@ -129,7 +129,7 @@ int fl_record_traces(int iz, int every, int max_traces);
 int fl_get_traces(float *host, int max_traces);
 
 /* nsteps steps it0+1 .. it0+nsteps of the reference loop (model.c:71-88): before step
- * it0+1+k, src[k] is added to pc and qc at iSource.  Steps are captured in HIP graphs
+ * it0+1+k, src[k] is added to pc and qc at iSource.  Fused steps are captured in HIP graphs
  * of graph_chunk steps (0: no graph) and replayed.  The instantiated graph is kept and
  * replayed by later calls with the same chunk, tiles, traces and source cell (any it0 and
  * nsteps): only the first such call pays for capture and instantiation. */
