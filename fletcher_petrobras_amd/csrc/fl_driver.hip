@@ -550,10 +550,9 @@ static int device_records(const ModelSrc &src, int cm, int sx, int sy, int sz, i
 
 // ------------------------------------------------------------------ launch plumbing
 // Workgroups of the step kernel resident on one CU: the LDS rings (6 staged planes and 5
-// Dx planes of ty+8 rows) against 160 KB, and the waves per SIMD the kernel is built for
-// (step_waves: 4 for FP32, 6 for the other forms with 8- or 12-row tiles).
-// Workgroups of the step kernel resident on one CU: limited by their LDS and by the waves
-// per SIMD their registers allow (step_waves, pair_waves in the kernels).
+// Dx planes of ty+8 rows; fewer with early_d2, where the waves are the limit) against 160
+// KB, and the waves per SIMD the kernel is built for (step_waves: 4 for FP32, 6 for the
+// other forms with 8- or 12-row tiles; pair_waves: 3).
 static int resident_per_cu(int ty, int cm, bool pair)
 {
     if (pair) {  // use_pair(cm, ty, ..): StepLds2

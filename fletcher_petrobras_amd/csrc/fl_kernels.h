@@ -227,6 +227,16 @@ __device__ __forceinline__ float der2_lds(const float *p, int s, float d2inv)
                d2inv);
 }
 
+// Both derivatives along one axis from the same neighbours (c the own value), each sum as above.
+template <bool SC>
+__device__ __forceinline__ void der12_lds(const float *p, int s, float c, float dinv, float d2inv, float &d1, float &d2)
+{
+    const float a1 = p[s], b1 = p[-s], a2 = p[2 * s], b2 = p[-2 * s], a3 = p[3 * s], b3 = p[-3 * s];
+    const float a4 = p[4 * s], b4 = p[-4 * s];
+    d1 = fd1<SC>(a1 - b1, a2 - b2, a3 - b3, a4 - b4, dinv);
+    d2 = fd2<SC>(c, a1 + b1, a2 + b2, a3 + b3, a4 + b4, d2inv);
+}
+
 // q[0..8] = values at z-4..z+4
 template <bool SC = true>
 __device__ __forceinline__ float der1_q(const float *q, float dinv)

@@ -14,7 +14,8 @@
 //              ring (10 slots) is addressed statically: the steady loop is unrolled 10
 //              times, one copy per ring phase, so planes advance without register moves.
 //   LDS        a ring of 6 staged planes of pc, qc (tile + 4-cell halo): plane f for Dx, Dy
-//              and the queues, plane z = f-4 for Dxx, Dyy, plane f+1 being written;
+//              and the queues, plane z = f-4 for Dxx, Dyy, plane f+1 being written (2 planes
+//              where Dxx, Dyy are formed at plane f, early_d2);
 //              a ring of 5 planes of Dx over the tile rows plus the 4-row y halo, from which
 //              Dxy(z) = Der1_y(Dx) is read (der1der1/sample.h:57-62, 83-88).
 // With the rings every plane needs a single barrier: nothing written in a step is read
@@ -306,10 +307,26 @@ __device__ __forceinline__ void decode_rec(const CoefRec<CM> &r, int fld, Coef &
     }
 }
 
-template <int TY>
+// Whether Dxx and Dyy are formed at the input plane f, from the neighbours that Dx and Dy read, and
+// kept in 5-slot register queues until f is the output plane four steps later; formed at
+// the output plane otherwise, from its staged plane.  The first way reads the staged plane
+// once a step instead of twice (34 instead of 50 LDS values a lane), needs two staged planes
+// instead of six, and has every LDS address static, for 15 more VGPRs.  Taken where they
+// are there, at 4 waves per SIMD (step_waves): 4- and 16-row tiles and FP32 on 8 rows, whose
+// steps are bound by the wave's chain of LDS reads and sums.  Arrays of 128^3 FP32 24.9 -> 22.9
+// us, 160^3 42.6 -> 40.1, 180^3 68.5 -> 62.6, 200^3 82.7 -> 79.5, 100^3 FP16 15.8 -> 14.7, FP16
+// recompute 16.6 -> 15.2.  FP32 on 12 rows, for large grids bound by memory, lost 0.5% with
+// the stream hints (384^3 637 -> 640 us) and keeps the other way, as do the forms held to 80 VGPRs.
+template <int TY, int CM>
+constexpr bool early_d2()
+{
+    return TY == 4 || TY == 16 || (TY == 8 && CM == CM_F32);
+}
+
+template <int TY, bool EARLY>
 struct StepLds {
     static constexpr int HX = 40, HY = TY + 8;
-    float t[6][HY * HX * 2];  // staged levels: (row, column, field) of the tile + halo
+    float t[EARLY ? 2 : 6][HY * HX * 2];  // staged levels: (row, column, field) of the tile + halo
     float x[5][HY * 32 * 2];  // Dx: (row, tile column, field), tile rows + y halo
 };
 
@@ -337,7 +354,7 @@ __device__ __forceinline__ void unroll_phases(F &&fn, std::integer_sequence<int,
 // inputs) and its sign is restored by a negative dz scale (or a multiply by -1 when ISO).
 template <int TY, int CM, bool TWOPASS, bool ISO, int PCPOL>
 __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl, int tix, int tiy, int zc,
-                                          bool down, StepLds<TY> &s)
+                                          bool down, StepLds<TY, early_d2<TY, CM>()> &s)
 {
     constexpr int TX = 32, HX = 40, HY = TY + 8, NT = 64 * TY;
     constexpr int RW = 2 * HX;                 // floats per staged row (pairs)
@@ -468,6 +485,10 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
     float qc_[10], qx_[10], qy_[10];
 #pragma unroll
     for (int k = 0; k < 10; k++) qc_[k] = qx_[k] = qy_[k] = 0.0f;
+    constexpr bool EARLY = early_d2<TY, CM>();
+    float qa_[5], qb_[5];  // EARLY: Dxx, Dyy of planes f-4..f (plane j in slot j % 5)
+#pragma unroll
+    for (int k = 0; k < 5; k++) qa_[k] = qb_[k] = 0.0f;
     // output-plane streams loaded prefetch_steps() ahead, in NSETS register sets (the set of
     // step i is (i - 8) % NSETS; NSETS divides the 10 steps of an unrolled group)
     constexpr int PDK = prefetch_steps<CM>() > 0 ? prefetch_steps<CM>() : 1;
@@ -509,8 +530,8 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
         constexpr int PD = prefetch_steps<CM>() > 0 ? prefetch_steps<CM>() : 1;
         const int z = zlo + pout(i);  // output plane
         const int r6n = r6 == 5 ? 0 : r6 + 1, r5n = r5 == 4 ? 0 : r5 + 1;
-        float *const Tf = s.t[r6];
-        float *const Tz = s.t[r6 >= 4 ? r6 - 4 : r6 + 2];
+        float *const Tf = s.t[EARLY ? SET : r6];
+        float *const Tz = s.t[EARLY ? 0 : r6 >= 4 ? r6 - 4 : r6 + 2];
         float *const Xf = s.x[r5];
         float *const Xz = s.x[r5n];
         const uint32_t so_o = (uint32_t)pout(i) * pb8;
@@ -534,8 +555,15 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
             for (int m = 0; m < NH; m++) gxh[m] = dvh_[SET][m];
         }
         const float *cp = Tf + ow + CW;
-        float nc = cp[0];
-        if constexpr (!TWOPASS) {
+        float nc = cp[0], nxx = 0.f, nyy = 0.f;
+        constexpr bool D2 = EARLY && XW != 0;
+        if constexpr (D2 && TWOPASS) {
+            nxx = der2_lds<!ISO>(cp, 2, a.dxxinv);
+            nyy = der2_lds<!ISO>(cp, RW, a.dyyinv);
+        } else if constexpr (D2) {
+            der12_lds<!ISO>(cp, 2, nc, a.dxinv, a.dxxinv, nx, nxx);
+            der12_lds<!ISO>(cp, RW, nc, a.dyinv, a.dyyinv, ny, nyy);
+        } else if constexpr (!TWOPASS) {
             nx = der1_lds<!ISO>(cp, 2, a.dxinv);
             ny = der1_lds<!ISO>(cp, RW, a.dyinv);
         }
@@ -557,16 +585,27 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
         qc_[ins] = nc;
         qx_[ins] = nx;
         qy_[ins] = ny;
+        if constexpr (D2) {
+            fl_pin(nxx);
+            fl_pin(nyy);
+            qa_[GEN ? 4 : PH % 5] = nxx;
+            qb_[GEN ? 4 : PH % 5] = nyy;
+        }
 
         float dxx = 0.f, dyy = 0.f, dxy = 0.f;
         if constexpr (OUT) {
-            const float *zp = Tz + ow + CW;
-            dxx = der2_lds<!ISO>(zp, 2, a.dxxinv);
-            dyy = der2_lds<!ISO>(zp, RW, a.dyyinv);
+            if constexpr (EARLY) {
+                dxx = qa_[GEN ? 0 : (PH + 1) % 5];
+                dyy = qb_[GEN ? 0 : (PH + 1) % 5];
+            } else {
+                const float *zp = Tz + ow + CW;
+                dxx = der2_lds<!ISO>(zp, 2, a.dxxinv);
+                dyy = der2_lds<!ISO>(zp, RW, a.dyyinv);
+            }
             dxy = der1_lds<!ISO>(Xz + oxw + CX, XW2, a.dyinv);
         }
         // next plane into the ring from its set, then the set refilled SA planes ahead
-        if (i + 1 <= nz + 7) stage(ic<(SET + 1) % SA>{}, s.t[r6n]);
+        if (i + 1 <= nz + 7) stage(ic<(SET + 1) % SA>{}, s.t[EARLY ? 1 - SET : r6n]);
         if (i + 1 + SA <= nz + 7) fetch(ic<(SET + 1) % SA>{}, i + 1 + SA);
         if constexpr (TWOPASS) {
             if (i + 2 <= nz + 7) fetch_dv(ic<SET>{}, i + 2);
@@ -640,6 +679,13 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
                 qx_[k] = qx_[k + 1];
                 qy_[k] = qy_[k + 1];
             }
+            if constexpr (EARLY) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    qa_[k] = qa_[k + 1];
+                    qb_[k] = qb_[k + 1];
+                }
+            }
         }
         r6 = r6n;
         r5 = r5n;
@@ -680,6 +726,14 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
             },
             std::make_integer_sequence<int, 10>{});
     }
+    // planes i-4 .. i-1 of the Dxx, Dyy queues (slots 4, 0, 1, 2: i = 8 mod 10) into slots 0-3
+    if constexpr (EARLY) {
+        const float a4 = qa_[4], b4 = qb_[4];
+        qa_[3] = qa_[2]; qb_[3] = qb_[2];
+        qa_[2] = qa_[1]; qb_[2] = qb_[1];
+        qa_[1] = qa_[0]; qb_[1] = qb_[0];
+        qa_[0] = a4; qb_[0] = b4;
+    }
     // the rest (i even here), queues shifted after each plane, two steps per round so that
     // the register sets keep their parity
     for (; i + 1 <= nz + 7; i += 2) {
@@ -709,7 +763,7 @@ template <int TY, int CM, bool TWOPASS, bool ISO, bool HINTS>
 __global__ __launch_bounds__(64 * TY) __attribute__((amdgpu_waves_per_eu(step_waves<TY, CM>())))
 void tti_step(const StepArgs a)
 {
-    __shared__ StepLds<TY> s;
+    __shared__ StepLds<TY, early_d2<TY, CM>()> s;
     const StepCtl ctl = step_ctl(a);
     if (a.run && blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0)
         a.run[1 - a.par] = a.run[a.par] + 1;
