@@ -573,14 +573,14 @@ static bool use_pair(int cm, int ty, bool twopass)
 
 // z chunk depth for `tiles` tile columns per plane over nzu planes: the chunk count that
 // minimises (rounds of the `slots` resident workgroups) x (planes a workgroup streams,
-// zt + lead).
-static int chunk_of(long long tiles, int nzu, long long slots, int lead)
+// zt + lead), with chunks of at least zmin planes.
+static int chunk_of(long long tiles, int nzu, long long slots, int lead, int zmin = 8)
 {
     double best = 1e300;
     int bz = nzu;
     for (int nzc = 1; nzc <= 64; nzc++) {
         const int zt = (nzu + nzc - 1) / nzc;
-        if (zt < 8 && nzc > 1) break;
+        if (zt < zmin && nzc > 1) break;
         const int n = (nzu + zt - 1) / zt;
         const long long rounds = (tiles * n + slots - 1) / slots;
         const double cost = (double)rounds * (zt + lead);
