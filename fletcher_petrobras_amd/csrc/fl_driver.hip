@@ -796,7 +796,8 @@ static int launch_step(StepArgs a, int it_host, hipStream_t s)
         const int nzu = D.sz - 2 * D.bord;
         // filling the ring costs a workgroup about as long as two planes; chunks of a single plane
         // and more, so that small grids spread over the chip (against eight and more: 53 x 51 x 48
-        // array 48.2 -> 12.5 us a step, 77 x 75 x 72 49.1 -> 23.6, 105 x 103 x 100 48.7 -> 33.7; the same from 128^3 up)
+        // array 48.2 -> 12.5 us a step, 77 x 75 x 72 49.1 -> 23.6, 105 x 103 x 100 48.7 -> 33.7;
+        // the same from 128^3 up)
         d.zt = chunk_of((long long)d.ntx * d.nty, nzu, (long long)std::max(g_cus, 1) * DX_PER_CU, 2, 1);
         d.nblk = d.ntx * d.nty * ((nzu + d.zt - 1) / d.zt);
         d.trace = nullptr;
