@@ -603,7 +603,11 @@ static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
 //   marching: rounds of resident workgroups x (zt + 0.46 x 8 lead planes) x the time of a plane
 //     step, 0.45 + 0.038 per wave on the CU (0.71 + 0.044 with both fields per lane): a wave's
 //     own chain of LDS reads and sums, and the issue slots of the others; the last round
-//     with the waves it has;
+//     with the waves it has.  Where Dxx, Dyy are formed at the input plane (early_d2)
+//     0.5 + 0.026, while the step's least bytes are at most 600 MB (FP32 and FP32 recompute)
+//     or 300 MB (the 16-bit forms): beyond, one 16-row workgroup a CU streams slower than several
+//     lower ones (FP16 232 x 240 x 228 cells 132 us against 118, block floating point 302 x 322 x
+//     312 299 against 265, FP32 376^3 732 against 700);
 //   memory: the step's bytes, the x-y halo and (8 planes a chunk) the z halo, at 6.2 TB/s.
 // Fitted on 15 grids from 28^3 to 376^3 updated cells in FP32, FP32 recompute, FP16, block
 // floating point and the two-pass form, every shape timed: the shape it picks takes 1.0% more
@@ -624,17 +628,19 @@ static double shape_us(const std::vector<GridDims> &g, int bord, int ty, int zt,
 {
     const bool pair = use_pair(cm, ty, twopass);
     const int res = resident_per_cu(ty, cm, pair), waves = pair ? ty / 2 : ty;
-    double items = 0, bytes = 0;
+    double items = 0, bytes = 0, least = 0;
     const double per = 24 + coef_count(cm) * coef_elem(cm) + (twopass ? 32 : 0);
     for (const GridDims &d : g) {
         const int nx = d.sx - 2 * bord, ny = d.sy - 2 * bord, nz = d.sz - 2 * bord;
         const int nzc = (nz + zt - 1) / zt;
         items += (double)tiles_x(d.sx, bord) * ((ny + ty - 1) / ty) * nzc;
+        least += (double)nx * ny * nz * per;
         bytes += (double)nx * ny * nz * (per + 64.0 * (2.1 * nzc / nz + 1.1 / ty));
     }
     const double cus = std::max(1, g_cus / 8), n8 = std::ceil(items / 8);  // per XCD
     const double full = std::floor(n8 / (cus * res)), rest = std::ceil((n8 - full * cus * res) / cus);
-    const double t0 = pair ? 0.71 : 0.45, tw = pair ? 0.044 : 0.038, steps = zt + 0.46 * 8;
+    const bool early = !pair && early_d2(ty, cm) && least <= ((cm == CM_F32 || cm == CM_F32R) ? 600e6 : 300e6);
+    const double t0 = pair ? 0.71 : early ? 0.5 : 0.45, tw = pair ? 0.044 : early ? 0.026 : 0.038, steps = zt + 0.46 * 8;
     double march = full * steps * (t0 + tw * waves * res);
     if (rest > 0) march += steps * (t0 + tw * waves * rest);
     return std::pow(std::pow(march, 4.5) + std::pow(bytes / 6.2e6, 4.5), 1 / 4.5);

@@ -317,10 +317,9 @@ __device__ __forceinline__ void decode_rec(const CoefRec<CM> &r, int fld, Coef &
 // us, 160^3 42.6 -> 40.1, 180^3 68.5 -> 62.6, 200^3 82.7 -> 79.5, 100^3 FP16 15.8 -> 14.7, FP16
 // recompute 16.6 -> 15.2.  FP32 on 12 rows, for large grids bound by memory, lost 0.5% with
 // the stream hints (384^3 637 -> 640 us) and keeps the other way, as do the forms held to 80 VGPRs.
-template <int TY, int CM>
-constexpr bool early_d2()
+constexpr bool early_d2(int ty, int cm)
 {
-    return TY == 4 || TY == 16 || (TY == 8 && CM == CM_F32);
+    return ty == 4 || ty == 16 || (ty == 8 && cm == CM_F32);
 }
 
 template <int TY, bool EARLY>
@@ -354,7 +353,7 @@ __device__ __forceinline__ void unroll_phases(F &&fn, std::integer_sequence<int,
 // inputs) and its sign is restored by a negative dz scale (or a multiply by -1 when ISO).
 template <int TY, int CM, bool TWOPASS, bool ISO, int PCPOL>
 __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl, int tix, int tiy, int zc,
-                                          bool down, StepLds<TY, early_d2<TY, CM>()> &s)
+                                          bool down, StepLds<TY, early_d2(TY, CM)> &s)
 {
     constexpr int TX = 32, HX = 40, HY = TY + 8, NT = 64 * TY;
     constexpr int RW = 2 * HX;                 // floats per staged row (pairs)
@@ -485,7 +484,7 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
     float qc_[10], qx_[10], qy_[10];
 #pragma unroll
     for (int k = 0; k < 10; k++) qc_[k] = qx_[k] = qy_[k] = 0.0f;
-    constexpr bool EARLY = early_d2<TY, CM>();
+    constexpr bool EARLY = early_d2(TY, CM);
     float qa_[5], qb_[5];  // EARLY: Dxx, Dyy of planes f-4..f (plane j in slot j % 5)
 #pragma unroll
     for (int k = 0; k < 5; k++) qa_[k] = qb_[k] = 0.0f;
@@ -763,7 +762,7 @@ template <int TY, int CM, bool TWOPASS, bool ISO, bool HINTS>
 __global__ __launch_bounds__(64 * TY) __attribute__((amdgpu_waves_per_eu(step_waves<TY, CM>())))
 void tti_step(const StepArgs a)
 {
-    __shared__ StepLds<TY, early_d2<TY, CM>()> s;
+    __shared__ StepLds<TY, early_d2(TY, CM)> s;
     const StepCtl ctl = step_ctl(a);
     if (a.run && blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0)
         a.run[1 - a.par] = a.run[a.par] + 1;

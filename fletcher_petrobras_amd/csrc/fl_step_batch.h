@@ -86,7 +86,7 @@ __global__ __launch_bounds__(PAIR ? 32 * TY : 64 * TY)
 __attribute__((amdgpu_waves_per_eu(PAIR ? pair_waves<TY>() : batch_waves<TY, CM>())))
 void tti_step_batch(const BatchArgs b, const ShotDev *__restrict__ shots, const int *__restrict__ item_shot)
 {
-    __shared__ std::conditional_t<PAIR, StepLds2<TY>, StepLds<TY, early_d2<TY, CM>()>> s;
+    __shared__ std::conditional_t<PAIR, StepLds2<TY>, StepLds<TY, early_d2(TY, CM)>> s;
     const int k = uni(b.run[b.par]);
     if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) b.run[1 - b.par] = k + 1;
     const int it = uni(b.run[RUN_IT_BASE]) + 1 + k;
