@@ -67,6 +67,7 @@ def lib():
         "fl_get_precision": (i, []),
         "fl_set_sync": (i, [i]),
         "fl_set_tiles": (i, [i, i]),
+        "fl_set_auto_tiles": (i, []),
         "fl_set_stream_hints": (i, [i]),
         "fl_set_tile_strip": (i, [i]),
         "fl_batch_set_persistent": (i, [i]),
@@ -99,6 +100,7 @@ def lib():
         "fl_bytes_per_cell": (i, []),
         "fl_batch_create": (i, [i, vp, i, f, f, f, f, i]),
         "fl_batch_set_tiles": (i, [i, i]),
+        "fl_batch_set_auto_tiles": (i, []),
         "fl_batch_get_tiles": (i, [C.c_void_p, C.c_void_p]),
         "fl_batch_run": (i, [i, i, _f32p, i, i, i]),
         "fl_batch_get_field": (i, [i, i, _f32p]),
@@ -456,6 +458,10 @@ class Driver:
     def set_tiles(self, ty, zt):
         _check(self.L.fl_set_tiles(ty, zt))
 
+    def set_auto_tiles(self):
+        """Tile rows and chunk depth left to the grid's size and form (the initial state)."""
+        _check(self.L.fl_set_auto_tiles())
+
     def tiles(self):
         a, b = C.c_int(), C.c_int()
         self.L.fl_get_tiles(C.byref(a), C.byref(b))
@@ -573,6 +579,9 @@ class Batch:
 
     def set_tiles(self, ty, zt):
         _check(self.L.fl_batch_set_tiles(ty, zt))
+
+    def set_auto_tiles(self):
+        _check(self.L.fl_batch_set_auto_tiles())
 
     def set_persistent(self, wgs):
         """0: one workgroup per item; 1: the persistent form over the resident workgroups;

@@ -59,7 +59,8 @@ extern "C" void fl_clear_error(void)
 // ------------------------------------------------------------------ helpers
 // ------------------------------------------------------------------ state
 struct Tiles {
-    int ty = 12, zt = 0;  // zt 0: chunk_depth's choice for the grid; (12, 0): pick_shape's
+    bool any = true;      // rows and depth left to pick_shape: the default, until fl_set_tiles
+    int ty = 12, zt = 0;  // zt 0: the depth that pick_shape (12 rows) or chunk_depth takes for these rows
     int hints = 0;        // streaming cache hints of the z-marching step (fl_set_stream_hints)
     int sw = 0;           // tile columns per strip (fl_set_tile_strip); 0: strip_width's choice
     int pair = 1;         // both fields per lane for the forms that have it (fl_set_lane_pairs)
@@ -83,7 +84,7 @@ struct Device {
     float *src_tab = nullptr;  // source samples of the current multi-step run
     int src_cap = 0;
     long long bytes = 0;
-    int auto_form = -1;     // variant and lane layout that the default tiles below are for
+    int auto_form = -1;     // variant, lane layout and row setting that pick_shape's tiles below are for
     int auto_ty = 0, auto_zt = 0;
 };
 
@@ -598,8 +599,8 @@ static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
     return std::max(1, std::min(std::min(chunk_of(tiles, nzu, slots, 8), nzu), ztmax));
 }
 
-// Tile rows and chunk depth of the default setting (12 rows, depth 0) for a set of grids stepped
-// together.  The modelled time of a shape, in us, is the 4.5-norm of
+// Tile rows and chunk depth of the default setting for a set of grids stepped together, or, with
+// 12 rows asked for, their depth.  The modelled time of a shape, in us, is the 4.5-norm of
 //   marching: rounds of resident workgroups x (zt + 0.46 x 8 lead planes) x the time of a plane
 //     step, 0.45 + 0.038 per wave on the CU (0.71 + 0.044 with both fields per lane): a wave's
 //     own chain of LDS reads and sums, and the issue slots of the others; the last round
@@ -646,7 +647,7 @@ static double shape_us(const std::vector<GridDims> &g, int bord, int ty, int zt,
     return std::pow(std::pow(march, 4.5) + std::pow(bytes / 6.2e6, 4.5), 1 / 4.5);
 }
 
-static Shape pick_shape(const std::vector<GridDims> &g, int bord, int cm, bool twopass)
+static Shape pick_shape(const std::vector<GridDims> &g, int bord, int cm, bool twopass, bool any)
 {
     int nzu = 0, ztmax = 1 << 30;
     for (const GridDims &d : g) {
@@ -659,7 +660,7 @@ static Shape pick_shape(const std::vector<GridDims> &g, int bord, int cm, bool t
     double least = shape_us(g, bord, best.ty, best.zt, cm, twopass);
     if (!has_pair_form(cm)) least *= 0.98;
     for (int ty : {4, 8, 12, 16})
-        for (int nzc = 1; nzc <= 64; nzc++) {
+        for (int nzc = 1; nzc <= 64 && (any || ty == 12); nzc++) {
             const int zt = std::min((nzu + nzc - 1) / nzc, ztmax);
             if (zt < 2 && nzc > 1) break;
             const double t = shape_us(g, bord, ty, zt, cm, twopass);
@@ -681,9 +682,9 @@ static Shape grid_shape()
         const long long tiles = (long long)tiles_x(D.sx, D.bord) * ((D.sy - 2 * D.bord + g_tiles.ty - 1) / g_tiles.ty);
         return {g_tiles.ty, chunk_depth(tiles, nz, g_tiles.ty, cm, ztmax)};
     }
-    const int form = 2 * g_variant + g_tiles.pair;
+    const int form = 4 * g_variant + 2 * g_tiles.pair + g_tiles.any;
     if (D.auto_form != form) {
-        const Shape s = pick_shape({{D.sx, D.sy, D.sz}}, D.bord, cm, g_variant == FL_VARIANT_TWOPASS);
+        const Shape s = pick_shape({{D.sx, D.sy, D.sz}}, D.bord, cm, g_variant == FL_VARIANT_TWOPASS, g_tiles.any);
         D.auto_form = form;
         D.auto_ty = s.ty;
         D.auto_zt = s.zt;
@@ -1137,8 +1138,17 @@ extern "C" int fl_set_tiles(int ty, int zt)
     if (ty != 4 && ty != 8 && ty != 12 && ty != 16)
         return fail(FL_ERR_ARG, "tile rows must be 4, 8, 12 or 16 (got %d)", ty);
     if (zt < 0) return fail(FL_ERR_ARG, "zt must be >= 0");
+    g_tiles.any = false;
     g_tiles.ty = ty;
     g_tiles.zt = zt;
+    return FL_OK;
+}
+
+extern "C" int fl_set_auto_tiles(void)
+{
+    g_tiles.any = true;
+    g_tiles.ty = Tiles().ty;
+    g_tiles.zt = Tiles().zt;
     return FL_OK;
 }
 
@@ -1632,7 +1642,7 @@ extern "C" int fl_autotune(int steps, const char *cache_path)
     const Tiles keep = g_tiles;
     double best = 1e30;
     Tiles bt = keep;
-    const Shape model = pick_shape({{D.sx, D.sy, D.sz}}, D.bord, D.cm, g_variant == FL_VARIANT_TWOPASS);
+    const Shape model = pick_shape({{D.sx, D.sy, D.sz}}, D.bord, D.cm, g_variant == FL_VARIANT_TWOPASS, true);
     // two passes over the candidates, the fastest single measurement wins: one pass
     // leaves the early candidates timed while the clocks still ramp.  Each is timed with
     // and without the streaming hints.
@@ -1643,6 +1653,7 @@ extern "C" int fl_autotune(int steps, const char *cache_path)
         std::vector<int> depths = zt_candidates(std::min(D.sz - 2 * D.bord, max_zt(D.px, D.sy)));
         if (cty == model.ty) depths.push_back(model.zt);
         for (int czt : depths) {
+            g_tiles.any = false;
             g_tiles.ty = cty;
             g_tiles.zt = czt;
             g_tiles.hints = ch;

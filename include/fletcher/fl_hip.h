@@ -63,11 +63,12 @@ int fl_get_precision(void);
 int fl_set_sync(int on);           /* 1 (default): DRIVER_Propagate waits for the step */
 
 /* Tile shape of the z-marching kernel: ty rows (4, 8, 12 or 16) of 32 cells, z chunks of
- * zt planes.  zt 0 selects the chunk depth that fits whole rounds of resident workgroups
- * to the grid; (12, 0), the default, leaves both rows and depth to the grid's size and form.
- * Results are identical for every shape.  fl_get_tiles returns the shape in use on the
- * initialised grid. */
+ * zt planes.  zt 0 selects the chunk depth for these rows by the grid (whole rounds of resident
+ * workgroups).  fl_set_auto_tiles, the state before any fl_set_tiles, leaves both rows and
+ * depth to the grid's size and form.  Results are identical for every shape.  fl_get_tiles
+ * returns the shape in use on the initialised grid. */
 int fl_set_tiles(int ty, int zt);
+int fl_set_auto_tiles(void);
 int fl_get_tiles(int *ty, int *zt);
 
 /* Streaming cache hints of the z-marching step (fused and two-pass variants): 1 loads and
@@ -185,7 +186,8 @@ typedef struct {
 
 int fl_batch_create(int nshots, const fl_shot_t *shots, int bord, float dx, float dy, float dz,
                     float dt, int precision);
-int fl_batch_set_tiles(int ty, int zt);
+int fl_batch_set_tiles(int ty, int zt);  /* as fl_set_tiles, fl_set_auto_tiles */
+int fl_batch_set_auto_tiles(void);
 /* Launch form of the batched step (no reference counterpart).  0 (default): one workgroup
  * per (shot, tile) item.  Otherwise the persistent form: the resident workgroups (at most
  * wgs of them when wgs > 1) take the items of their slice of the work list from a ticket
