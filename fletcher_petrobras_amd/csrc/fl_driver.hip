@@ -177,7 +177,7 @@ extern "C" int fl_bytes_per_cell(void)
 // memory, which the runtime splits into one copy a row: 10 us a row, 330 of the 340 ms of a
 // 128^3 DRIVER_Initialize, now 10 ms; a 384^3 field came down at 17 GB/s in pageable
 // copies (13 ms), now in 4.6 ms.  Kept between transfers, released by DRIVER_Finalize and
-// fl_batch_destroy.
+// fl_batch_destroy, and by fl_ref64_destroy where neither a grid nor a batch is set up.
 constexpr size_t PIPE_BYTES = 16u << 20;
 struct Pipe {
     char *pin[2] = {nullptr, nullptr}, *dev[2] = {nullptr, nullptr};
