@@ -306,20 +306,6 @@ void fl_pack_recompute32(int64_t n, const float *vpz, const float *vsv, const fl
     }
 }
 
-void fl_interleave32(int64_t n, int nk, const float *const *src, float *dst)
-{
-#pragma omp parallel for schedule(static)
-    for (int64_t i = 0; i < n; i++)
-        for (int k = 0; k < nk; k++) dst[i * nk + k] = src[k][i];
-}
-
-void fl_interleave16(int64_t n, int nk, const uint16_t *const *src, uint16_t *dst)
-{
-#pragma omp parallel for schedule(static)
-    for (int64_t i = 0; i < n; i++)
-        for (int k = 0; k < nk; k++) dst[i * nk + k] = src[k][i];
-}
-
 void fl_copy_parallel(void *dst, const void *src, size_t bytes)
 {
     const size_t part = 1u << 20;
