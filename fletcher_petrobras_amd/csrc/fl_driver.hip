@@ -551,8 +551,8 @@ static int device_records(const ModelSrc &src, int cm, int sx, int sy, int sz, i
 
 // ------------------------------------------------------------------ launch plumbing
 // Workgroups of the step kernel resident on one CU: the LDS rings (6 staged planes and 5
-// Dx planes of ty+8 rows; fewer with early_d2, where the waves are the limit) against 160
-// KB, and the waves per SIMD the kernel is built for (step_waves: 4 for FP32, 6 for the
+// Dx planes of ty+8 rows; 2 staged planes with early_d2, where the waves are the limit with
+// either) against 160 KB, and the waves per SIMD the kernel is built for (step_waves: 4 for FP32, 6 for the
 // other forms with 8- or 12-row tiles; pair_waves: 3).
 static int resident_per_cu(int ty, int cm, bool pair)
 {
@@ -607,17 +607,21 @@ static int chunk_depth(long long tiles, int nzu, int ty, int cm, int ztmax)
 //     with the waves it has.  Where Dxx, Dyy are formed at the input plane (early_d2)
 //     0.5 + 0.026, while the step's least bytes are at most 600 MB (FP32 and FP32 recompute)
 //     or 300 MB (the 16-bit forms): beyond, one 16-row workgroup a CU streams slower than several
-//     lower ones (FP16 232 x 240 x 228 cells 132 us against 118, block floating point 302 x 322 x
-//     312 299 against 265, FP32 376^3 732 against 700);
+//     lower ones (arrays of 240 x 248 x 236 FP16 136 us against 122, 310 x 330 x 320 block floating
+//     point 296 against 266 and FP16 348 against 310, 384^3 FP32 732 against 700);
 //   memory: the step's bytes, the x-y halo and (8 planes a chunk) the z halo, at 6.2 TB/s.
-// Fitted on 15 grids from 28^3 to 376^3 updated cells in FP32, FP32 recompute, FP16, block
-// floating point and the two-pass form, every shape timed: the shape it picks takes 1.0% more
-// than the fastest one on average, 7% at most.  Against 12 rows with chunk_depth (the
-// default before) it is up to twice as fast on small grids (52 x 44 x 40 FP32 15.2 -> 9.0 us,
-// 120^3 28.0 -> 26.0, q16r 27.3 -> 24.4), 10-20% on middle ones (160^3 FP32 58.0 -> 47.7,
-// q16r 248^3 155.7 -> 137.8) and equal or up to 10% faster on large ones; a one-field-per-lane
-// shape has to promise 2% over the 12-row one to replace it (376^3 FP32: 32x16x63 took 735 us
-// against 704; two-pass: 32x16x94 1270 against 1245).
+// Checked against every shape on 15 arrays from 36^3 to 384^3 in FP32, FP32 recompute, FP16, block
+// floating point and the two-pass form: the shape it picks takes 2.3% more than the fastest one on
+// average (2.1, 5.5, 0.7, 1.1 and 1.9% by form).  It is off most where one 16-row chunk of the whole
+// column, or of half of it, keeps every workgroup resident: 341 x 297 x 373 FP32 488 us (16 x 61)
+// against 426 (16 x 365) and FP32 recompute 402 against 333, 310 x 330 x 320 422 against 375 and 340
+// against 292, FP32 recompute beyond the line on 240 x 248 x 236 131 against 115 and 256^3 154 against
+// 136; all others are within 8.1%.  The two-pass form (96 B a cell at the lines) is within 3.5% from 150^3 up.
+// Against 12 rows with chunk_depth: 64 x 60 x 56 FP32 15.1 -> 8.7 us, 128^3 27.5 -> 22.5, 168^3
+// 57.6 -> 44.1, 256^3 198 -> 178; block floating point 128^3 28.9 -> 22.5, 256^3 142 -> 124; equal on
+// 384^3 FP32.  A one-field-per-lane shape has to promise 2% over the 12-row one to replace it (384^3
+// FP32: 32x16x63 takes 732 us against 700; two-pass: 32x16x94 1266 against 1246).  With 12 rows asked
+// for, the depth is the model's too: 64 x 60 x 56 FP32 15.1 -> 9.3 us, 160^3 55.3 -> 56.9, mostly equal.
 struct Shape {
     int ty, zt;
 };

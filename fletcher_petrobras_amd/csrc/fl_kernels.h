@@ -432,8 +432,10 @@ __device__ __forceinline__ f4 dercross_h(H h, float dinv)
 // leapfrog keep the reference's association order: the results are those of the reference's
 // loop, bit for bit.
 //
-// Bound by VALU issue (573 operations a cell, none of them fused, in the reference's order)
-// with the LDS close behind: a lane reads 131 16-byte values a plane, 1048 bytes a cell with
+// Bound by both units at two waves a SIMD, neither of them full: on a 192 x 240 x 216 array the VALU
+// is busy 65% of the time (573 operations a cell, none of them fused, in the reference's order), the
+// LDS 59% (half of that bank conflicts of the 16-byte reads), and waves wait 37% of theirs; HBM traffic is
+// 2.7 TB/s.  A lane reads 131 16-byte values a plane, 1048 bytes a cell with
 // both fields, where one cell a lane with both fields read 217 pairs, 1736 bytes.  That form,
 // which also waited for the next plane's loads at the end of each plane, took 414 us on a
 // 192 x 240 x 216 array and 2141 us on 384^3; this one 217 and 1182 us (the VALU operations
@@ -593,7 +595,7 @@ void direct_dercross(const DirectArgs a)
 // lane idles on rows that are not multiples of 64, and the blocks of a plane stay on one XCD
 // (xcd_remap), whose L2 holds the shared halo rows.  The four volumes are read back only
 // after the whole pass: stored non-temporally (default policy: 183 against 171 us a two-pass step).
-// Measured: 224 x 208 x 192 array 74 -> 53 us, 384^3 491 -> 298 us (4.6 TB/s).  Rows a thread: 4 is
+// Measured: 224 x 208 x 192 array 74 -> 51 us, 384^3 491 -> 294 us (4.6 TB/s).  Rows a thread: 4 is
 // as fast as 8 and 16 on large arrays and faster on small ones (two-pass step on 104 x 110 x 100:
 // 29.4, 31.3, 36.0 us with 4, 8, 16).
 //

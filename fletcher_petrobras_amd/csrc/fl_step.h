@@ -742,11 +742,13 @@ __device__ __forceinline__ void step_tile(const StepArgs &a, const StepCtl &ctl,
     if (i <= nz + 7) step(ic<0>{}, ic<2>{}, ic<1>{}, ic<1>{}, ic<0>{}, ic<0>{}, ic<0>{}, i, false);
 }
 
-// Waves per SIMD the register allocator is asked for.  With 8-row tiles the LDS rings
-// (51 KB per workgroup) allow three workgroups per CU, with 12-row tiles (63 KB) two:
-// 6 waves per SIMD, <= 80 VGPRs, which the 16-bit and recompute forms meet.  The FP32
-// records keep 4 waves (83 VGPRs): a 6-wave build spills only outside the steady loop but
-// measured no faster at 344^3.  4- and 16-row tiles are held to 4 waves per SIMD by their LDS.
+// Waves per SIMD the register allocator is asked for.  With 8-row tiles of the 16-bit and recompute
+// forms the LDS rings (50 KiB per workgroup) allow three workgroups per CU, with 12-row tiles
+// (62.5 KiB) two: 6 waves per SIMD, <= 80 VGPRs, which these forms meet (FP16 and block floating
+// point with one value spilled).  The FP32 records keep 4 waves (84 VGPRs on 12 rows): a 6-wave
+// build spills only outside the steady loop but measured no faster at 344^3.  4- and 16-row tiles,
+// and FP32 on 8 rows, form Dxx, Dyy early: their rings need 22.5, 45 and 30 KiB, so it is the registers
+// (92-105 VGPRs with the two queues) that hold them to 4 waves per SIMD.
 // FL_STEP_WAVES overrides the 8- and 12-row value at build time.
 template <int TY, int CM>
 constexpr int step_waves()
